@@ -413,10 +413,10 @@ def setup_c5(vqx, torch, L, whole_tiles=False, M=2048):
 def setup_c5_linear_mx(vqx, torch, L, M=2048):
     """C5 through the reference's own op: quantized_ops::linear_mx with the
     operands convert_pt2e writes (bf16 code indices [11008, 4096], the 16 NF4
-    levels as weight_code, bf16 scales [11008, 64]).  The first call packs the
-    weight (cached); each step is one torch op call, whose fused kernel is
-    what the HIP events time (with the op's host dispatch hidden behind the
-    previous launch)."""
+    levels as weight_code, bf16 scales [11008, 64]).  The first call decodes
+    the weight (cached); each step is one torch op call, whose dense product
+    is what the HIP events time (with the op's host dispatch hidden behind
+    the previous launch)."""
     g = torch.Generator().manual_seed(4)
     N, K = 11008, 4096
     Ac = torch.randn(M, K, generator=g).to(torch.bfloat16)
@@ -431,11 +431,11 @@ def setup_c5_linear_mx(vqx, torch, L, M=2048):
         Q.linear_mx(A, idx, None, weight_scale=scale, weight_code=code, block_size=64)
         return 0
 
-    launch()  # packs the weight once
+    launch()  # decodes the weight once
     return [launch], dict(
         name=f"C5 via quantized_ops::linear_mx on convert-format operands: A bf16 [{M},4096], weight = bf16 NF4 "
              f"indices [11008,4096] + weight_code (16 bf16 levels) + bf16 weight_scale [11008,64], block 64 -> bf16; "
-             f"the fused dequant MFMA kernel (weight packed once, cached)",
+             f"the dense MFMA kernel on the weight's bf16 decode (decoded once, cached)",
         elements=M * N, flops=2 * M * N * K, bytes=M * K * 2 + N * K // 2 + N * K // 64 * 4 + M * N * 2,
         bound="mfma", dtype="bf16", cpu=cpu_c5(torch, Ac, N), keep=(A, idx, scale, code))
 
@@ -551,8 +551,8 @@ def setup_c6_mxnf4_linear(vqx, torch, L, M=2048, N=11008, K=4096):
     quantized_ops::linear_mx: nf4_6 activation indices with input_code and
     fp8_e5m3-grid input_scale per 64 along K, a convert-format nf4_6 weight
     (16-entry weight_code, weight_scale per 64): the activation's decode pass,
-    then the packed-weight product (graph replay of one call; the weight is
-    packed once, cached)."""
+    then the dense product (graph replay of one call; the weight is decoded
+    once, cached)."""
     g = torch.Generator().manual_seed(8)
     bs = 64
     code = torch.tensor([-31., -22., -16., -12., -9., -6., -3., 0., 2., 5., 8., 10., 14., 17., 22., 31.],

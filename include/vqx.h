@@ -430,6 +430,22 @@ int vqx_mx_matmul(const VqxMxOperand* a, const VqxMxOperand* b, const uint16_t* 
                   int64_t batch, int64_t M, int64_t N, int64_t K, vqx_stream_t stream);
 
 /*
+ * The product of two plain bf16 matrices with K contiguous, where
+ * linear_mx / matmul_mx end once their operands are decoded (src/vc/ops/
+ * quantized.py:328-333, 400-406): out[b][M][N] = a[b] . b[b]^T (+ bias), fp32
+ * accumulation, bf16 out (contiguous).  a: [M][K] rows lda elements apart,
+ * b: [N][K] rows ldb apart; items a_batch_stride / b_batch_stride elements
+ * apart (0: shared); both 16-byte aligned, the strides multiples of 8, one
+ * item under 4 GiB.  bias: bf16 [N] or NULL.  K % 64 == 0; any M and N.
+ * workspace (16-byte aligned): vqx_dense_matmul_workspace_size bytes let a
+ * product with few tiles split K; with less (or NULL) it runs whole tiles.
+ */
+int vqx_dense_matmul(const uint16_t* a, int64_t lda, int64_t a_batch_stride, const uint16_t* b, int64_t ldb,
+                     int64_t b_batch_stride, const uint16_t* bias, uint16_t* out, int64_t batch, int64_t M,
+                     int64_t N, int64_t K, void* workspace, int64_t workspace_bytes, vqx_stream_t stream);
+int vqx_dense_matmul_workspace_size(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t* bytes);
+
+/*
  * The operand decode of linear_mx / matmul_mx (src/vc/ops/quantized.py:
  * 313-326, 388-398) on its own: x (a VqxMxOperand: k_major = 1 for
  * [rows][K], 0 for [K][rows]) decoded to dense bf16 in the same layout,

@@ -356,6 +356,32 @@ int vqx_mx_matmul(const VqxMxOperand* a, const VqxMxOperand* b, const uint16_t* 
                  N, K, (hipStream_t)stream);
 }
 
+int vqx_dense_matmul(const uint16_t* a, int64_t lda, int64_t a_batch_stride, const uint16_t* b, int64_t ldb,
+                     int64_t b_batch_stride, const uint16_t* bias, uint16_t* out, int64_t batch, int64_t M,
+                     int64_t N, int64_t K, void* workspace, int64_t workspace_bytes, vqx_stream_t stream) {
+  g_err[0] = 0;
+  if (!a || !b || !out) return set_error(kErrInvalid, "dense_matmul: null buffer");
+  if (!dense_gemm_takes(batch, M, N, K))
+    return set_error(kErrInvalid, "dense_matmul: batch %lld M %lld N %lld K %lld (K %% 64 == 0 needed)", (long long)batch,
+                     (long long)M, (long long)N, (long long)K);
+  if (!aligned(a, 16) || !aligned(b, 16) || lda % 8 || ldb % 8 || a_batch_stride % 8 || b_batch_stride % 8)
+    return set_error(kErrInvalid, "dense_matmul: operands must be 16-byte aligned, strides multiples of 8");
+  if (lda < K || ldb < K || a_batch_stride < 0 || b_batch_stride < 0)
+    return set_error(kErrInvalid, "dense_matmul: row stride below K or negative batch stride");
+  // each item is addressed with 32-bit byte offsets
+  if (2 * ((M - 1) * lda + K) >= ((int64_t)1 << 32) || 2 * ((N - 1) * ldb + K) >= ((int64_t)1 << 32))
+    return set_error(kErrInvalid, "dense_matmul: one batch item spans more than 4 GiB");
+  return dense_gemm(a, lda, a_batch_stride, b, ldb, b_batch_stride, bias, out, batch, M, N, K, workspace,
+                    workspace_bytes, (hipStream_t)stream);
+}
+
+int vqx_dense_matmul_workspace_size(int64_t batch, int64_t M, int64_t N, int64_t K, int64_t* bytes) {
+  g_err[0] = 0;
+  if (!bytes) return set_error(kErrInvalid, "dense_matmul_workspace_size: null result");
+  *bytes = dense_gemm_takes(batch, M, N, K) ? dense_gemm_workspace(batch, M, N, K) : 0;
+  return kOk;
+}
+
 int vqx_mx_operand_decode(const VqxMxOperand* x, int64_t batch, int64_t rows, int64_t K, uint16_t* out,
                           vqx_stream_t stream) {
   g_err[0] = 0;

@@ -220,6 +220,13 @@ int mx_gemm(const MxOperand& a, const MxOperand& b, const uint16_t* bias, uint16
             int64_t N, int64_t K, hipStream_t st);
 int mx_decode(const MxOperand& x, int64_t batch, int64_t rows, int64_t K, uint16_t* out, hipStream_t st);
 
+// vqx_dense_gemm.hip: a [M][K] and b [N][K] plain bf16, strides in elements
+bool dense_gemm_takes(int64_t batch, int64_t M, int64_t N, int64_t K);
+int64_t dense_gemm_workspace(int64_t batch, int64_t M, int64_t N, int64_t K);
+int dense_gemm(const uint16_t* a, int64_t lda, int64_t a_bstride, const uint16_t* b, int64_t ldb, int64_t b_bstride,
+               const uint16_t* bias, uint16_t* out, int64_t batch, int64_t M, int64_t N, int64_t K, void* workspace,
+               int64_t workspace_bytes, hipStream_t st);
+
 // vqx_sparse.hip
 struct CsrDecode {
   const void* B;        // [nb, br, bc], dtype b_dtype (float tags or kU8)

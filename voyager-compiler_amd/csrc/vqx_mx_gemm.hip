@@ -497,7 +497,7 @@ int launch_one(const MxOpArgs& a, const MxOpArgs& b, const uint16_t* bias, uint1
 
 // The tile, from measurement (LLaMA-7B shapes on one MI355X): 256 x 128
 // for products with N > 128 and K > 128 that still give every CU a tile
-// (the MXINT8 MLP linear: 253 against 282 us), else 128 x 128 (two
+// (2048 x 11008 x 4096: 253 against 282 us), else 128 x 128 (two
 // workgroups per CU: the attention products, K = 128 or N = 128, run 9% and
 // 6% faster on it).
 enum TileKind : int { kT128 = 0, kT256x128 = 1 };
@@ -603,6 +603,11 @@ int mx_gemm(const MxOperand& a, const MxOperand& b, const uint16_t* bias, uint16
   if (!out || !aligned(out, 8)) return set_error(kErrInvalid, "mx_gemm: out must be 8-byte aligned");
   if (bias && !aligned(bias, 8)) return set_error(kErrInvalid, "mx_gemm: bias must be 8-byte aligned");
   if (batch > INT32_MAX) return set_error(kErrInvalid, "mx_gemm: batch too large");
+  // nothing to decode and K contiguous on both sides: the dense product (from
+  // four of its 64-deep steps; below that its pipeline does not fill)
+  if (dec_of(a) == kPlain && dec_of(b) == kPlain && b.k_major && K >= 256 && dense_gemm_takes(batch, M, N, K))
+    return dense_gemm(static_cast<const uint16_t*>(a.data), a.ld, a.batch_stride, static_cast<const uint16_t*>(b.data),
+                      b.ld, b.batch_stride, bias, out, batch, M, N, K, nullptr, 0, stream);
   const MxOpArgs aa = args_of(a), bb = args_of(b);
   const int db = dec_of(b);
   const bool bk = b.k_major != 0;

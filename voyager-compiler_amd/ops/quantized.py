@@ -14,6 +14,7 @@ Ops beyond the reference's (packed storage is this build's own):
 
 import ctypes
 import math
+import threading
 import weakref
 from typing import List, Optional, Tuple
 
@@ -710,6 +711,14 @@ def _packed_weight(weight, weight_code, weight_scale, transposed):
     return None if entry.codes is None else (entry.codes, entry.scale, entry.levels)
 
 
+# Rows up to which an NF4 linear reads the packed 4-bit weight; above it runs
+# on the weight's cached bf16 decode.  At 16 rows the packed weight's smaller
+# traffic wins (4096 x 4096: 7.9 against 17.2 us, 11008 x 4096 19 against 26),
+# from 17 rows, where the packed product leaves its 16-row kernel, the dense
+# one (57 against 17 us, 61 against 24; at 2048 rows 209 against 172).
+_PACKED_ROWS = 16
+
+
 def _fusable(x, weight, bias, weight_scale, block_size, weight_code, transposed):
     """Whether the product of x with this weight can run fused: bf16
     activations, a 2-D bf16 index weight with a code table of at most 16
@@ -858,10 +867,41 @@ def _right_operand(b, code, scale, block_size, stored_kn):
 # probabilities of P V (one column tile).
 _FUSED_DECODE_MAX_TILES = 4
 _DECODED = {}
+# Bytes of cached decodes per device.  A linear that has another way (the
+# packed NF4 product, the decode inside the product) takes it rather than let
+# the cache pass a quarter of the device's memory; a weight's decode is given
+# back with the weight.
+_DECODED_SHARE = 4
+_DECODED_BYTES = {}
+_DECODED_LOCK = threading.Lock()
+_DEVICE_BYTES = {}
+
+
+def _nbytes(t):
+    return t.numel() * t.element_size()
+
+
+def _store_decoded(key, entry):
+    """Set (or with None drop) a cache entry, keeping the per-device total."""
+    with _DECODED_LOCK:
+        old = _DECODED.pop(key, None)
+        for e, sign in ((old, -1), (entry, 1)):
+            if e is not None:
+                d = e[2].device.index
+                _DECODED_BYTES[d] = _DECODED_BYTES.get(d, 0) + sign * _nbytes(e[2])
+        if entry is not None:
+            _DECODED[key] = entry
+
+
+def _decoded_fits(nbytes, device):
+    total = _DEVICE_BYTES.get(device.index)
+    if total is None:
+        total = _DEVICE_BYTES[device.index] = torch.cuda.get_device_properties(device).total_memory
+    return _DECODED_BYTES.get(device.index, 0) + nbytes <= total // _DECODED_SHARE
 
 
 def _release_decoded(key):
-    _DECODED.pop(key, None)
+    _store_decoded(key, None)
 
 
 def _mx_decoded(t, code, scale, block_size, kdim):
@@ -912,10 +952,11 @@ def _activation_decoded(x, code, scale, block_size):
     return _decode_operand(x, code, scale, block_size)
 
 
-def _decoded_weight(weight, code, scale, block_size, kdim):
+def _decoded_weight(weight, code, scale, block_size, kdim, bounded=False):
     """The bf16 decode of a convert-format weight, cached per weight tensor
     and rebuilt when the weight, its code or its scale change (version
-    counters), as the packed NF4 weight is."""
+    counters), as the packed NF4 weight is.  bounded: None instead of a new
+    entry that would take the cache past its share of the device's memory."""
     key = id(weight)
     deps = (weight, code, scale)
     versions = tuple(None if t is None else (t.data_ptr(), _lib.version_of(t)) for t in deps)
@@ -923,11 +964,77 @@ def _decoded_weight(weight, code, scale, block_size, kdim):
     if hit is not None and hit[1] == versions and all(
             (r is None and t is None) or (r is not None and r() is t) for r, t in zip(hit[0], deps)):
         return hit[2]
+    if bounded and hit is None and not _decoded_fits(_nbytes(weight), weight.device):
+        return None
     dense = _mx_decoded(weight, code, scale, block_size, kdim)
+    if torch.cuda.is_current_stream_capturing():
+        return dense  # part of the graph being captured (its memory pool): decoded again on each replay
+    # a later call may come on another stream: it finds the decode finished
+    torch.cuda.current_stream(weight.device).synchronize()
     if hit is None:
         weakref.finalize(weight, _release_decoded, key)
-    _DECODED[key] = (tuple(None if t is None else weakref.ref(t) for t in deps), versions, dense)
+    _store_decoded(key, (tuple(None if t is None else weakref.ref(t) for t in deps), versions, dense))
     return dense
+
+
+_DENSE_WS = {}
+
+
+def _dense_workspace_bytes(batch, M, N, K, device):
+    """Workspace vqx_dense_matmul needs to split K for this shape on
+    ``device`` (0: whole tiles), cached per shape."""
+    key = (batch, M, N, K, device.index)
+    n = _DENSE_WS.get(key)
+    if n is None:
+        if len(_DENSE_WS) >= 4096:
+            _DENSE_WS.clear()
+        got = ctypes.c_int64(0)
+        with torch.cuda.device(device):
+            _lib.call("vqx_dense_matmul_workspace_size", batch, M, N, K, ctypes.byref(got))
+        n = _DENSE_WS[key] = got.value
+    return n
+
+
+def _dense_linear(x2, w, bias):
+    """x2 [M, K] . w[N, K]^T (+ bias) on plain contiguous bf16 operands
+    through vqx_dense_matmul, launched on x2's current stream."""
+    M, K = x2.shape
+    N = w.shape[0]
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=x2.device)
+    ws_bytes = _dense_workspace_bytes(1, M, N, K, x2.device)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x2.device) if ws_bytes else None
+    _lib.call("vqx_dense_matmul", _lib.ptr(x2), K, 0, _lib.ptr(w), K, 0, _lib.ptr(bias), _lib.ptr(out), 1, M, N, K,
+              _lib.ptr(ws), ws_bytes, _lib.stream_of(x2))
+    return out
+
+
+def _dense_takes(M, N, K):
+    """Shapes vqx_dense_matmul takes: whole 64-deep steps, each operand under
+    4 GiB (its kernel addresses them with 32-bit byte offsets)."""
+    return K % 64 == 0 and K > 0 and M > 0 and N > 0 and 2 * M * K < 1 << 32 and 2 * N * K < 1 << 32
+
+
+def _dense_weight_linear(a, a_code, a_scale, w, w_code, w_scale, block_size, bias):
+    """A linear whose weight [N, K] is decoded once (cached) and whose
+    activations a [M, K] are decoded by the streaming pass, as one dense
+    product; None when the operands fall outside it.  At every M this beats
+    decoding the weight in the product's staging (1000 x 4096 x 4096 MXINT8
+    61 -> 45 us, 512 rows 56 -> 28 us of product)."""
+    M, K = a.shape
+    if w.dim() != 2 or w.shape[1] != K or not _dense_takes(M, w.shape[0], K) or a.device != w.device:
+        return None
+    if not (_mx_side_ok(a, a_code, a_scale, block_size, -1) and _mx_side_ok(w, w_code, w_scale, block_size, -1)):
+        return None
+    if bias is not None and (bias.dtype != torch.bfloat16 or tuple(bias.shape) != (w.shape[0],)
+                             or bias.device != a.device):
+        return None
+    if w_code is not None or w_scale is not None:
+        w = _decoded_weight(w, w_code, w_scale, block_size, -1, bounded=True)
+        if w is None:
+            return None
+    if a_code is not None or a_scale is not None:
+        a = _mx_decoded(a, a_code, a_scale, block_size, -1)
+    return _dense_linear(_aligned16(a), _aligned16(w), None if bias is None else bias.contiguous())
 
 
 def _mx_product(a, a_code, a_scale, b, b_code, b_scale, block_size, b_stored_kn, bias, b_static=False):
@@ -1014,7 +1121,19 @@ def linear_mx(input, weight, bias=None, *, input_scale=None, weight_scale=None, 
     transposed = weight_layout == "ck"
     dense = None
     x = None
-    if weight_code is not None and weight_code.numel() <= 16:
+    packable = weight_code is not None and weight_code.numel() <= 16
+    few_rows = packable and input.dim() > 0 and input.numel() <= _PACKED_ROWS * input.shape[-1]
+    if not few_rows and not transposed and _coded(input_code, input_scale, weight_code, weight_scale) \
+            and input.dim() > 0 and input.shape[-1] > 0:
+        # [M, K] rows against the weight decoded once
+        K = input.shape[-1]
+        if input_scale is None or tuple(input_scale.shape[:-1]) == tuple(input.shape[:-1]):
+            s = None if input_scale is None else input_scale.reshape(-1, input_scale.shape[-1])
+            dense = _dense_weight_linear(input.reshape(-1, K), input_code, s, weight, weight_code, weight_scale,
+                                         block_size, bias)
+            if dense is not None:
+                dense = dense.reshape(*input.shape[:-1], dense.shape[-1])
+    if dense is None and packable:
         x = _activation_decoded(input, input_code, input_scale, block_size)
         if _fusable(x, weight, bias, weight_scale, block_size, weight_code, transposed):
             dense = _fused_linear(x, weight, bias, weight_scale, weight_code, transposed)
