@@ -396,8 +396,9 @@ int vqx_nf4_pack_weight(const void* weight, int32_t w_dtype, const void* scale, 
  *                scale_batch_stride multiples of 8).
  * batch_stride / scale_batch_stride: elements between batch items (0: the
  * same matrix for every item).  data 16-byte aligned, ld and batch_stride
- * multiples of 8; block_size a power of two >= 8; code: bf16, code_len
- * 1..256 entries.
+ * multiples of 8 (any, 2-byte aligned, in vqx_mx_matmul_any and
+ * vqx_mx_operand_rows); block_size a power of two >= 8; code: bf16, code_len 1..256
+ * entries.
  */
 typedef struct VqxMxOperand {
   const void* data;
@@ -430,6 +431,13 @@ int vqx_mx_matmul(const VqxMxOperand* a, const VqxMxOperand* b, const uint16_t* 
                   int64_t batch, int64_t M, int64_t N, int64_t K, vqx_stream_t stream);
 
 /*
+ * vqx_mx_matmul on K-major operands (b.k_major = 1) of any K >= 8, alignment
+ * and strides: a 2-byte aligned row is read in 16-byte loads all the same.
+ */
+int vqx_mx_matmul_any(const VqxMxOperand* a, const VqxMxOperand* b, const uint16_t* bias, uint16_t* out,
+                      int64_t batch, int64_t M, int64_t N, int64_t K, vqx_stream_t stream);
+
+/*
  * The product of two plain bf16 matrices with K contiguous, where
  * linear_mx / matmul_mx end once their operands are decoded (src/vc/ops/
  * quantized.py:328-333, 400-406): out[b][M][N] = a[b] . b[b]^T (+ bias), fp32
@@ -456,6 +464,17 @@ int vqx_dense_matmul_workspace_size(int64_t batch, int64_t M, int64_t N, int64_t
  */
 int vqx_mx_operand_decode(const VqxMxOperand* x, int64_t batch, int64_t rows, int64_t K, uint16_t* out,
                           vqx_stream_t stream);
+
+/*
+ * The same decode with its rows in the order and length a product wants: out
+ * [batch][rows][out_ld] with K last (k_last = 1, out_ld >= K) or
+ * [batch][K][out_ld] (k_last = 0, out_ld >= rows), zeros past the last value
+ * of a row.  An x of the other order is turned on the way.  Any K and rows;
+ * x any alignment; out 16-byte aligned, and out_ld a multiple of 8 unless x
+ * is turned.
+ */
+int vqx_mx_operand_rows(const VqxMxOperand* x, int64_t batch, int64_t rows, int64_t K, int32_t k_last, uint16_t* out,
+                        int64_t out_ld, vqx_stream_t stream);
 
 /*
  * quantized_ops::filter_outlier (src/vc/ops/quantized.py:532-630, with

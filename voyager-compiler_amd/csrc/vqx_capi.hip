@@ -353,7 +353,15 @@ int vqx_mx_matmul(const VqxMxOperand* a, const VqxMxOperand* b, const uint16_t* 
   static_assert(sizeof(VqxMxOperand) == sizeof(MxOperand), "VqxMxOperand and MxOperand differ");
   if (!a || !b) return set_error(kErrInvalid, "mx_matmul: null operand descriptor");
   return mx_gemm(*reinterpret_cast<const MxOperand*>(a), *reinterpret_cast<const MxOperand*>(b), bias, out, batch, M,
-                 N, K, (hipStream_t)stream);
+                 N, K, false, (hipStream_t)stream);
+}
+
+int vqx_mx_matmul_any(const VqxMxOperand* a, const VqxMxOperand* b, const uint16_t* bias, uint16_t* out,
+                      int64_t batch, int64_t M, int64_t N, int64_t K, vqx_stream_t stream) {
+  g_err[0] = 0;
+  if (!a || !b) return set_error(kErrInvalid, "mx_matmul: null operand descriptor");
+  return mx_gemm(*reinterpret_cast<const MxOperand*>(a), *reinterpret_cast<const MxOperand*>(b), bias, out, batch, M,
+                 N, K, true, (hipStream_t)stream);
 }
 
 int vqx_dense_matmul(const uint16_t* a, int64_t lda, int64_t a_batch_stride, const uint16_t* b, int64_t ldb,
@@ -386,7 +394,19 @@ int vqx_mx_operand_decode(const VqxMxOperand* x, int64_t batch, int64_t rows, in
                           vqx_stream_t stream) {
   g_err[0] = 0;
   if (!x) return set_error(kErrInvalid, "mx_decode: null operand descriptor");
-  return mx_decode(*reinterpret_cast<const MxOperand*>(x), batch, rows, K, out, (hipStream_t)stream);
+  if (K % 8) return set_error(kErrInvalid, "mx_decode: K (%lld) must be a multiple of 8", (long long)K);
+  if (!x->k_major && rows % 8)
+    return set_error(kErrInvalid, "mx_decode: an N-major operand needs a multiple of 8 columns");
+  return mx_decode(*reinterpret_cast<const MxOperand*>(x), batch, rows, K, out, x->k_major ? K : rows, false,
+                   (hipStream_t)stream);
+}
+
+int vqx_mx_operand_rows(const VqxMxOperand* x, int64_t batch, int64_t rows, int64_t K, int32_t k_last, uint16_t* out,
+                        int64_t out_ld, vqx_stream_t stream) {
+  g_err[0] = 0;
+  if (!x) return set_error(kErrInvalid, "mx_rows: null operand descriptor");
+  return mx_decode(*reinterpret_cast<const MxOperand*>(x), batch, rows, K, out, out_ld,
+                   (x->k_major != 0) != (k_last != 0), (hipStream_t)stream);
 }
 
 int vqx_nf4_pack_weight(const void* weight, int32_t w_dtype, const void* scale, int32_t s_dtype, int64_t N,

@@ -119,15 +119,37 @@ __device__ __forceinline__ float bf_hi(uint32_t w) { return u2f(w & 0xFFFF0000u)
 struct Raw {
   u32x4 v[4];
   u32x4 s;  // K-major: s[q] low half = scale of chunk q; N-major: the 8 columns' scales
-  bool in;  // the chunks lie inside K (past K they are zero and must decode to zero)
+  int in;   // k values of the chunks inside K (values past K must decode to zero)
 };
+
+// 16 bytes from a 2-byte aligned address (rows whose length is not a multiple
+// of 8 values): one load instruction, which takes any alignment.
+__device__ __forceinline__ u32x4 load16_any(const char* p) {
+  u32x4 v;
+  __builtin_memcpy(&v, __builtin_assume_aligned(p, 2), 16);
+  return v;
+}
+
+// The values of v from element n (0..7) on, zeros behind them.
+__device__ __forceinline__ u32x4 shift_down(u32x4 v, int n) {
+  const uint64_t lo = v.x | ((uint64_t)v.y << 32), hi = v.z | ((uint64_t)v.w << 32);
+  const int b = 16 * (n & 3);
+  const uint64_t l = n & 4 ? hi : lo, h = n & 4 ? 0 : hi;
+  const uint64_t rl = b ? (l >> b) | (h << (64 - b)) : l, rh = h >> b;
+  return {(uint32_t)rl, (uint32_t)(rl >> 32), (uint32_t)rh, (uint32_t)(rh >> 32)};
+}
+
+// Mask of dword j (values 2 j, 2 j + 1) of a chunk with n valid values.
+__device__ __forceinline__ uint32_t valid_mask(int n, int j) {
+  return n >= 2 * j + 2 ? 0xFFFFFFFFu : (n == 2 * j + 1 ? 0xFFFFu : 0u);
+}
 
 // K-major staging of ROWS tile rows (A, or B stored [N][K]) by THREADS
 // threads: chunk q of thread t is chunk t % 8 of tile row t / 8 + q THREADS / 8.
 // Loads are never skipped (a branch around a load makes the compiler wait for
 // every load in flight at the join): past the last row the last row is read,
-// past K the last chunk, and in a checked step the chunk is zeroed after the
-// load.  Addresses are a uniform base (the batch item) plus 32-bit byte
+// past K the last 8 values, and in a checked step the values past K are zeroed
+// after the decode.  K and the row stride may be any (K >= 8).  Addresses are a uniform base (the batch item) plus 32-bit byte
 // offsets; LDS addresses are precomputed.
 template <int D, int ROWS, int THREADS>
 struct KMajor {
@@ -156,18 +178,20 @@ struct KMajor {
   }
   template <bool CHECK>
   __device__ __forceinline__ void load(Raw& x, int ks, int K) {
-    int k = ks * kTK + (threadIdx.x & 7) * 8;
-    x.in = true;
+    const int k = ks * kTK + (threadIdx.x & 7) * 8;
+    int kl = k;
+    x.in = 8;
     if constexpr (CHECK) {
-      x.in = k < K;
-      k = x.in ? k : K - 8;
+      x.in = K - k;  // 8 or more: all
+      kl = k < K - 8 ? k : K - 8;
     }
-    const uint32_t kb = 2u * (uint32_t)(k - (int)(threadIdx.x & 7) * 8);
+    const uint32_t kb = 2u * (uint32_t)(kl - (int)(threadIdx.x & 7) * 8);
+    const int ksc = CHECK && k >= K ? kl : k;  // a chunk wholly past K takes any scale
 #pragma unroll
     for (int q = 0; q < kCh; ++q) {
-      x.v[q] = *reinterpret_cast<const u32x4*>(base + (off[q] + kb));
+      x.v[q] = load16_any(base + (off[q] + kb));
       if constexpr (D == kScale || D == kCodeScale)
-        x.s[q] = *reinterpret_cast<const uint16_t*>(sbase + (soff[q] + 2u * (uint32_t)(k >> sh)));
+        x.s[q] = *reinterpret_cast<const uint16_t*>(sbase + (soff[q] + 2u * (uint32_t)(ksc >> sh)));
     }
   }
   // decode and write to the stage; in a checked step chunks past K are
@@ -177,11 +201,14 @@ struct KMajor {
 #pragma unroll
     for (int q = 0; q < kCh; ++q) {
       const float s = bf_lo(x.s[q]);
-      u32x4 d;
+      u32x4 d, v = x.v[q];
+      if constexpr (CHECK) {
+        if (x.in < 8) v = shift_down(v, (8 - x.in) & 7);  // loaded from K - 8 on
+      }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        d[j] = decode2<D>(x.v[q][j], s, s, tab);
-        if constexpr (CHECK) d[j] = x.in ? d[j] : 0u;
+        d[j] = decode2<D>(v[j], s, s, tab);
+        if constexpr (CHECK) d[j] &= valid_mask(x.in, j);
       }
       *reinterpret_cast<u32x4*>(stage + lds[q]) = d;
     }
@@ -222,9 +249,9 @@ struct NMajor {
   __device__ __forceinline__ void load(Raw& x, int ks, int K) {
     if (!active()) return;
     int k = ks * kTK + ((int)threadIdx.x / kOct) * 4;
-    x.in = true;
+    x.in = 8;
     if constexpr (CHECK) {
-      x.in = k < K;  // K % 8 == 0: the four rows are all in or all out
+      x.in = k < K ? 8 : 0;  // K % 8 == 0: the four rows are all in or all out
       k = x.in ? k : K - 4;
     }
     const uint32_t r0 = (uint32_t)k * ldb + coff;
@@ -446,41 +473,152 @@ __global__ __launch_bounds__((TM == 128 && TN == 128) ? 256 : 512, 2) void mx_ge
                    m0 + wm * S::kWRows, n0 + wn * 64);
 }
 
-// The decode of one operand into dense bf16 in its own layout: the pass the
-// host runs ahead of the product for an operand that many output tiles read.
-// Item b of the operand is [R][C] (row stride o.ld), out is [items][R][C]
-// contiguous; K-major: C = K, blocks along C; N-major: R = K, blocks along R.
-// Each thread decodes 8 consecutive values of a row per iteration.
-template <int D, bool KMAJ>
-__global__ __launch_bounds__(256) void mx_decode_kernel(MxOpArgs o, uint16_t* __restrict__ out, int R, int C,
-                                                        uint32_t chunks) {
-  __shared__ uint16_t tab[D >= kCode ? 2 * kCodeSpan : 1];
+// Decode passes: an operand that many output tiles read, decoded once into
+// dense bf16 ahead of the product.  The code table in LDS has one entry per
+// index from -len - 1 to len, the first and last (clamped to by everything
+// outside, NaN too) decoding to NaN: built from 2 len + 2 reads, where the
+// product kernel's table by bit pattern (2054 entries, fewer instructions per
+// lookup) took most of the pass (333 x 11008 activations 8.0 us).
+struct CodeLookup {
+  const uint16_t* tab;
+  float lo, hi;
+  int off;
+  __device__ __forceinline__ uint32_t operator()(uint32_t h) const {
+    const float v = __builtin_fminf(__builtin_fmaxf(u2f(h << 16), lo), hi);
+    return tab[(int)v + off];
+  }
+};
+
+template <int D>
+__device__ __forceinline__ CodeLookup make_lookup(uint16_t* tab, const MxOpArgs& o) {
+  const int len = o.code_len;
   if constexpr (D >= kCode) {
-    build_code_table<256>(tab, o.code, o.code_len);
+    for (int e = threadIdx.x; e < 2 * len + 2; e += 256) {
+      const int i = e - len - 1;
+      tab[e] = i >= -len && i < len ? o.code[i < 0 ? i + len : i] : (uint16_t)0x7FC0u;
+    }
     __syncthreads();
   }
-  const uint32_t cpr = (uint32_t)C / 8u;
+  return {tab, -(float)(len + 1), (float)len, len + 1};
+}
+
+template <int D>
+__device__ __forceinline__ uint32_t decode_pair(uint32_t w, float s0, float s1, const CodeLookup& lk) {
+  if constexpr (D == kPlain) {
+    return w;
+  } else if constexpr (D == kScale) {
+    return pack_bf16x2(bf_lo(w) * s0, bf_hi(w) * s1);
+  } else {
+    const uint32_t lo = lk(w & 0xFFFFu), hi = lk(w >> 16);
+    if constexpr (D == kCode) return lo | (hi << 16);
+    else return pack_bf16x2(u2f(lo << 16) * s0, u2f(hi << 16) * s1);
+  }
+}
+
+// Up to n values from p, zeros behind them.
+__device__ __forceinline__ u32x4 load8(const uint16_t* p, int n) {
+  if (n >= 8) return load16_any(reinterpret_cast<const char*>(p));
+  u32x4 v = {0u, 0u, 0u, 0u};
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    if (e < n) v[e >> 1] |= (uint32_t)p[e] << (16 * (e & 1));
+  return v;
+}
+
+// Decode in the operand's own layout.  Item b of the operand is [R][C] (row
+// stride o.ld, any alignment), out is [items][R][CP] contiguous with CP >= C
+// a multiple of 8, zeros past C; KMAJ: C = K, blocks along C; else R = K,
+// blocks along R.  Each thread decodes 8 consecutive values of a row per
+// iteration.
+template <int D, bool KMAJ>
+__global__ __launch_bounds__(256) void mx_decode_kernel(MxOpArgs o, uint16_t* __restrict__ out, int R, int C, int CP,
+                                                        uint32_t chunks) {
+  __shared__ uint16_t tab[D >= kCode ? 2 * kMaxCode + 2 : 1];
+  const CodeLookup lk = make_lookup<D>(tab, o);
+  const uint32_t cpr = (uint32_t)CP / 8u;
   for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < chunks; i += gridDim.x * 256u) {
     const uint32_t row = i / cpr;  // over all items
     const int c = (int)(i - row * cpr) * 8;
     const uint32_t bi = row / (uint32_t)R;
     const int r = (int)(row - bi * (uint32_t)R);
-    const u32x4 v = ld_nt(reinterpret_cast<const u32x4*>(o.data + (int64_t)bi * o.bstride + (int64_t)r * o.ld + c));
-    u32x4 d;
-    if constexpr (KMAJ) {
-      float s = 1.0f;
-      if constexpr (D == kScale || D == kCodeScale)
-        s = bf_lo(o.scale[(int64_t)bi * o.sbstride + (int64_t)r * o.sld + (c >> o.bs_shift)]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) d[j] = decode2<D>(v[j], s, s, tab);
-    } else {
+    const int n = C - c;  // values of the chunk inside the row
+    u32x4 d = {0u, 0u, 0u, 0u};
+    if (n > 0) {
+      const u32x4 v = load8(o.data + (int64_t)bi * o.bstride + (int64_t)r * o.ld + c, n);
       u32x4 sc = {0u, 0u, 0u, 0u};
-      if constexpr (D == kScale || D == kCodeScale)
-        sc = *reinterpret_cast<const u32x4*>(o.scale + (int64_t)bi * o.sbstride + (int64_t)(r >> o.bs_shift) * o.sld + c);
+      float s = 1.0f;
+      if constexpr (D == kScale || D == kCodeScale) {
+        const uint16_t* sp = o.scale + (int64_t)bi * o.sbstride;
+        if constexpr (KMAJ) s = bf_lo(sp[(int64_t)r * o.sld + (c >> o.bs_shift)]);
+        else sc = load8(sp + (int64_t)(r >> o.bs_shift) * o.sld + c, n);
+      }
 #pragma unroll
-      for (int j = 0; j < 4; ++j) d[j] = decode2<D>(v[j], bf_lo(sc[j]), bf_hi(sc[j]), tab);
+      for (int j = 0; j < 4; ++j)
+        d[j] = decode_pair<D>(v[j], KMAJ ? s : bf_lo(sc[j]), KMAJ ? s : bf_hi(sc[j]), lk) & valid_mask(n, j);
     }
-    st_nt(reinterpret_cast<u32x4*>(out + (int64_t)row * C + c), d);
+    *reinterpret_cast<u32x4*>(out + (int64_t)row * CP + c) = d;
+  }
+}
+
+// Decode with a transpose: item b of the operand is [R][C] (row stride o.ld,
+// any alignment), out is [items][C][RP] contiguous with RP >= R, zeros past R.
+// SROW: the scales' blocks run along R (an N-major operand: R = K), one scale
+// row per block; else along C (a K-major weight laid out by rows of K).  A
+// workgroup turns a 64 x 64 tile: a thread loads 8 columns of two rows, pairs
+// them by column and writes 8 dwords to LDS (row c of the tile holds 64 r in
+// eight 16-byte slots, slot s at s ^ (c >> 3): at most two lanes a bank), then
+// four threads write each column's 128 bytes.
+template <int D, bool SROW>
+__global__ __launch_bounds__(256) void mx_turn_kernel(MxOpArgs o, uint16_t* __restrict__ out, int R, int C, int RP,
+                                                      int tr, int tc) {
+  __shared__ uint16_t tab[D >= kCode ? 2 * kMaxCode + 2 : 1];
+  __shared__ __attribute__((aligned(16))) uint32_t tile[64 * 32];
+  const CodeLookup lk = make_lookup<D>(tab, o);
+  const int b = blockIdx.x / (tr * tc), rem = blockIdx.x - b * (tr * tc);
+  const int r0 = rem / tc * 64, c0 = rem % tc * 64;
+  const uint16_t* data = o.data + (int64_t)b * o.bstride;
+  const uint16_t* scale = nullptr;
+  if constexpr (D == kScale || D == kCodeScale) scale = o.scale + (int64_t)b * o.sbstride;
+  const int rp = threadIdx.x >> 3, cc = (threadIdx.x & 7) * 8;  // row pair, first column in the tile
+  const int n = C - (c0 + cc);
+  u32x4 d[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int r = r0 + 2 * rp + h;
+    d[h] = u32x4{0u, 0u, 0u, 0u};
+    if (r < R && n > 0) {
+      const u32x4 v = load8(data + (int64_t)r * o.ld + c0 + cc, n);
+      u32x4 sc = {0u, 0u, 0u, 0u};
+      float s = 1.0f;
+      if constexpr (D == kScale || D == kCodeScale) {
+        if constexpr (SROW) sc = load8(scale + (int64_t)(r >> o.bs_shift) * o.sld + c0 + cc, n);
+        else s = bf_lo(scale[(int64_t)r * o.sld + ((c0 + cc) >> o.bs_shift)]);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) d[h][j] = decode_pair<D>(v[j], SROW ? bf_lo(sc[j]) : s, SROW ? bf_hi(sc[j]) : s, lk);
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    uint32_t* t = tile + (cc + 2 * j) * 32 + ((((uint32_t)rp >> 2) ^ ((uint32_t)cc >> 3)) << 2) + (rp & 3);
+    t[0] = __builtin_amdgcn_perm(d[1][j], d[0][j], 0x05040100u);
+    t[32] = __builtin_amdgcn_perm(d[1][j], d[0][j], 0x07060302u);
+  }
+  __syncthreads();
+  const int c = threadIdx.x >> 2;
+  if (c0 + c >= C) return;
+  uint16_t* orow = out + ((int64_t)b * C + c0 + c) * RP;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int s = (threadIdx.x & 3) * 2 + h, r = r0 + s * 8;
+    const u32x4 v = *reinterpret_cast<const u32x4*>(tile + c * 32 + ((s ^ (c >> 3)) << 2));
+    if (r + 8 <= RP) {
+      __builtin_memcpy(__builtin_assume_aligned(orow + r, 2), &v, 16);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (r + e < RP) orow[r + e] = (uint16_t)(v[e >> 1] >> (16 * (e & 1)));
+    }
   }
 }
 
@@ -539,13 +677,16 @@ int dec_of(const MxOperand& o) { return (o.code ? kCode : kPlain) | (o.scale ? k
 // 32-bit byte offsets from the item's base.
 constexpr int64_t kMaxItemBytes = (int64_t)1 << 32;
 
-int check_operand(const MxOperand& o, const char* name, bool k_major_only, int64_t K, int64_t cols) {
-  if (!o.data || !aligned(o.data, 16)) return set_error(kErrInvalid, "%s: data must be a 16-byte aligned pointer", name);
+// any: the operand may have any alignment and strides (else 16-byte aligned
+// data, strides and N-major scales, as the N-major staging reads them).
+int check_operand(const MxOperand& o, const char* name, bool k_major_only, int64_t K, int64_t cols, bool any = false) {
+  if (!o.data || !aligned(o.data, any ? 2 : 16))
+    return set_error(kErrInvalid, "%s: data must be a 16-byte aligned pointer", name);
   if (k_major_only && !o.k_major) return set_error(kErrInvalid, "%s: the left operand is K-major ([M][K])", name);
   const int64_t need = o.k_major ? K : cols;
-  if (o.ld < need || o.ld % 8) return set_error(kErrInvalid, "%s: ld %lld must be >= %lld and a multiple of 8", name,
-                                                (long long)o.ld, (long long)need);
-  if (o.batch_stride < 0 || o.batch_stride % 8)
+  if (o.ld < need || (!any && o.ld % 8)) return set_error(kErrInvalid, "%s: ld %lld must be >= %lld and a multiple of 8", name,
+                                                          (long long)o.ld, (long long)need);
+  if (o.batch_stride < 0 || (!any && o.batch_stride % 8))
     return set_error(kErrInvalid, "%s: batch_stride must be >= 0 and a multiple of 8", name);
   const int64_t span = o.k_major ? (cols - 1) * o.ld + K : (K - 1) * o.ld + cols;
   if (2 * span >= kMaxItemBytes)
@@ -563,7 +704,8 @@ int check_operand(const MxOperand& o, const char* name, bool k_major_only, int64
     if (o.k_major) {
       if (o.scale_ld < nkb) return set_error(kErrInvalid, "%s: scale_ld must be >= %lld", name, (long long)nkb);
     } else {
-      if (!aligned(o.scale, 16) || o.scale_ld < cols || o.scale_ld % 8 || o.scale_batch_stride % 8)
+      if (o.scale_ld < cols ||
+          (!any && (!aligned(o.scale, 16) || o.scale_ld % 8 || o.scale_batch_stride % 8)))
         return set_error(kErrInvalid,
                          "%s: N-major scales need a 16-byte aligned pointer, scale_ld >= %lld and strides that are "
                          "multiples of 8",
@@ -590,22 +732,23 @@ MxOpArgs args_of(const MxOperand& o) {
 }  // namespace
 
 int mx_gemm(const MxOperand& a, const MxOperand& b, const uint16_t* bias, uint16_t* out, int64_t batch, int64_t M,
-            int64_t N, int64_t K, hipStream_t stream) {
+            int64_t N, int64_t K, bool any, hipStream_t stream) {
   if (batch < 1 || M < 1 || N < 1 || K < 1) return set_error(kErrInvalid, "mx_gemm: empty product");
-  if (K % 8) return set_error(kErrInvalid, "mx_gemm: K (%lld) must be a multiple of 8", (long long)K);
+  if (!any && K % 8) return set_error(kErrInvalid, "mx_gemm: K (%lld) must be a multiple of 8", (long long)K);
+  if (any && (K < 8 || !b.k_major)) return set_error(kErrInvalid, "mx_gemm: K-major operands with K >= 8 needed");
   if (N % 4) return set_error(kErrInvalid, "mx_gemm: N (%lld) must be a multiple of 4", (long long)N);
   if (!b.k_major && N % 8) return set_error(kErrInvalid, "mx_gemm: an N-major right operand needs N %% 8 == 0");
   if (M > INT32_MAX || N > INT32_MAX || K > INT32_MAX) return set_error(kErrInvalid, "mx_gemm: dimension too large");
-  int rc = check_operand(a, "mx_gemm A", true, K, M);
+  int rc = check_operand(a, "mx_gemm A", true, K, M, any);
   if (rc) return rc;
-  rc = check_operand(b, "mx_gemm B", false, K, N);
+  rc = check_operand(b, "mx_gemm B", false, K, N, any);
   if (rc) return rc;
   if (!out || !aligned(out, 8)) return set_error(kErrInvalid, "mx_gemm: out must be 8-byte aligned");
   if (bias && !aligned(bias, 8)) return set_error(kErrInvalid, "mx_gemm: bias must be 8-byte aligned");
   if (batch > INT32_MAX) return set_error(kErrInvalid, "mx_gemm: batch too large");
   // nothing to decode and K contiguous on both sides: the dense product (from
   // four of its 64-deep steps; below that its pipeline does not fill)
-  if (dec_of(a) == kPlain && dec_of(b) == kPlain && b.k_major && K >= 256 && dense_gemm_takes(batch, M, N, K))
+  if (!any && dec_of(a) == kPlain && dec_of(b) == kPlain && b.k_major && K >= 256 && dense_gemm_takes(batch, M, N, K))
     return dense_gemm(static_cast<const uint16_t*>(a.data), a.ld, a.batch_stride, static_cast<const uint16_t*>(b.data),
                       b.ld, b.batch_stride, bias, out, batch, M, N, K, nullptr, 0, stream);
   const MxOpArgs aa = args_of(a), bb = args_of(b);
@@ -622,33 +765,58 @@ int mx_gemm(const MxOperand& a, const MxOperand& b, const uint16_t* bias, uint16
 }
 
 template <int D>
-int launch_decode(bool kmaj, const MxOpArgs& o, uint16_t* out, int R, int C, uint32_t chunks, hipStream_t stream) {
+int launch_decode(bool kmaj, const MxOpArgs& o, uint16_t* out, int R, int C, int CP, uint32_t chunks,
+                  hipStream_t stream) {
   const unsigned grid = grid_for(chunks, 256, 8);
   if (kmaj)
-    hipLaunchKernelGGL((mx_decode_kernel<D, true>), dim3(grid), dim3(256), 0, stream, o, out, R, C, chunks);
+    hipLaunchKernelGGL((mx_decode_kernel<D, true>), dim3(grid), dim3(256), 0, stream, o, out, R, C, CP, chunks);
   else
-    hipLaunchKernelGGL((mx_decode_kernel<D, false>), dim3(grid), dim3(256), 0, stream, o, out, R, C, chunks);
+    hipLaunchKernelGGL((mx_decode_kernel<D, false>), dim3(grid), dim3(256), 0, stream, o, out, R, C, CP, chunks);
   return check_launch("mx_decode_kernel");
 }
 
-int mx_decode(const MxOperand& x, int64_t batch, int64_t rows, int64_t K, uint16_t* out, hipStream_t stream) {
+template <int D>
+int launch_turn(bool srow, const MxOpArgs& o, uint16_t* out, int R, int C, int RP, int64_t batch, hipStream_t stream) {
+  const int tr = (RP + 63) / 64, tc = (C + 63) / 64;
+  const dim3 grid((unsigned)(batch * tr * tc));
+  if (srow) hipLaunchKernelGGL((mx_turn_kernel<D, true>), grid, dim3(256), 0, stream, o, out, R, C, RP, tr, tc);
+  else hipLaunchKernelGGL((mx_turn_kernel<D, false>), grid, dim3(256), 0, stream, o, out, R, C, RP, tr, tc);
+  return check_launch("mx_turn_kernel");
+}
+
+// x decoded into dense bf16: in its own layout (turn 0, rows padded with zeros
+// to out_ld, a multiple of 8), or with its two dims swapped (turn 1).
+int mx_decode(const MxOperand& x, int64_t batch, int64_t rows, int64_t K, uint16_t* out, int64_t out_ld, bool turn,
+              hipStream_t stream) {
   if (batch < 1 || rows < 1 || K < 1) return set_error(kErrInvalid, "mx_decode: empty operand");
-  if (K % 8) return set_error(kErrInvalid, "mx_decode: K (%lld) must be a multiple of 8", (long long)K);
-  if (!x.k_major && rows % 8)
-    return set_error(kErrInvalid, "mx_decode: an N-major operand needs a multiple of 8 columns");
-  int rc = check_operand(x, "mx_decode", false, K, rows);
+  int rc = check_operand(x, "mx_decode", false, K, rows, true);
   if (rc) return rc;
+  const int64_t R = x.k_major ? rows : K, C = x.k_major ? K : rows, ol = turn ? R : C;
   if (!out || !aligned(out, 16)) return set_error(kErrInvalid, "mx_decode: out must be 16-byte aligned");
-  const int64_t R = x.k_major ? rows : K, C = x.k_major ? K : rows;
-  const int64_t chunks = batch * R * (C / 8);
-  if (chunks > INT32_MAX || batch * R > INT32_MAX) return set_error(kErrInvalid, "mx_decode: operand too large");
+  if (out_ld < ol || (!turn && out_ld % 8))
+    return set_error(kErrInvalid, "mx_decode: out_ld %lld for rows of %lld", (long long)out_ld, (long long)ol);
+  if (R > INT32_MAX || C > INT32_MAX || out_ld > INT32_MAX - 64 || batch * R > INT32_MAX)
+    return set_error(kErrInvalid, "mx_decode: operand too large");
   const MxOpArgs o = args_of(x);
+  const int d = dec_of(x), iR = (int)R, iC = (int)C, il = (int)out_ld;
   const bool km = x.k_major != 0;
-  switch (dec_of(x)) {
-    case kPlain: return launch_decode<kPlain>(km, o, out, (int)R, (int)C, (uint32_t)chunks, stream);
-    case kScale: return launch_decode<kScale>(km, o, out, (int)R, (int)C, (uint32_t)chunks, stream);
-    case kCode: return launch_decode<kCode>(km, o, out, (int)R, (int)C, (uint32_t)chunks, stream);
-    default: return launch_decode<kCodeScale>(km, o, out, (int)R, (int)C, (uint32_t)chunks, stream);
+  if (turn) {
+    if (batch * ((out_ld + 63) / 64) * ((C + 63) / 64) > INT32_MAX)
+      return set_error(kErrInvalid, "mx_decode: operand too large");
+    switch (d) {
+      case kPlain: return launch_turn<kPlain>(!km, o, out, iR, iC, il, batch, stream);
+      case kScale: return launch_turn<kScale>(!km, o, out, iR, iC, il, batch, stream);
+      case kCode: return launch_turn<kCode>(!km, o, out, iR, iC, il, batch, stream);
+      default: return launch_turn<kCodeScale>(!km, o, out, iR, iC, il, batch, stream);
+    }
+  }
+  const int64_t chunks = batch * R * (out_ld / 8);
+  if (chunks > INT32_MAX) return set_error(kErrInvalid, "mx_decode: operand too large");
+  switch (d) {
+    case kPlain: return launch_decode<kPlain>(km, o, out, iR, iC, il, (uint32_t)chunks, stream);
+    case kScale: return launch_decode<kScale>(km, o, out, iR, iC, il, (uint32_t)chunks, stream);
+    case kCode: return launch_decode<kCode>(km, o, out, iR, iC, il, (uint32_t)chunks, stream);
+    default: return launch_decode<kCodeScale>(km, o, out, iR, iC, il, (uint32_t)chunks, stream);
   }
 }
 

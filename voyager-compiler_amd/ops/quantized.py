@@ -938,6 +938,36 @@ def _mx_decoded(t, code, scale, block_size, kdim):
     return out.transpose(-2, -1) if flipped else out
 
 
+def _mx_rows(t, code, scale, block_size, kdim, k_last=True, ld=None):
+    """t (bf16, contraction dim kdim = -1 or -2, scales along it) decoded to
+    dense bf16 rows of K (k_last) padded with zeros to ld, or rows of the
+    other dim, turned on the way when t is stored in the other order
+    (vqx_mx_operand_rows): [batch, rows, ld], batch dims flattened."""
+    lead = t.shape[:-2]
+    tt = t.transpose(-2, -1)
+    if t.is_contiguous():
+        m, flipped = t, False
+    elif tt.is_contiguous():
+        m, flipped = tt, True
+    else:
+        m, flipped = t.contiguous(), False
+    k_major = (kdim == -1) != flipped
+    R, C = m.shape[-2], m.shape[-1]
+    K, cols = (C, R) if k_major else (R, C)
+    sm = None
+    if scale is not None:
+        sm = (scale.transpose(-2, -1) if flipped else scale).contiguous()
+    batch = math.prod(lead)
+    op = _mx_operand(m, None if code is None else _code_bf16(code, t.device), sm, block_size, k_major, R * C, C,
+                     0 if sm is None else sm.shape[-2] * sm.shape[-1], 0 if sm is None else sm.shape[-1])
+    last, outer = (K, cols) if k_last else (cols, K)
+    ld = last if ld is None else ld
+    out = torch.empty(batch, outer, ld, dtype=torch.bfloat16, device=t.device)
+    _lib.call("vqx_mx_operand_rows", _lib.ctypes.byref(op), batch, cols, K, 1 if k_last else 0, _lib.ptr(out), ld,
+              _lib.stream_of(t))
+    return out
+
+
 def _activation_decoded(x, code, scale, block_size):
     """The left operand's decode ahead of the packed-weight product: the
     streaming decode pass when it takes the operand (bf16, scales along the
@@ -952,21 +982,21 @@ def _activation_decoded(x, code, scale, block_size):
     return _decode_operand(x, code, scale, block_size)
 
 
-def _decoded_weight(weight, code, scale, block_size, kdim, bounded=False):
-    """The bf16 decode of a convert-format weight, cached per weight tensor
-    and rebuilt when the weight, its code or its scale change (version
-    counters), as the packed NF4 weight is.  bounded: None instead of a new
-    entry that would take the cache past its share of the device's memory."""
-    key = id(weight)
-    deps = (weight, code, scale)
+def _cached_decode(form, deps, nbytes, make, bounded):
+    """make() for the weight deps[0] and the code / scale it decodes with,
+    cached per weight tensor and form, rebuilt when one of deps changes
+    (version counters).  bounded: None instead of a new entry that would take
+    the cache past its share of the device's memory."""
+    weight = deps[0]
+    key = (id(weight), form)
     versions = tuple(None if t is None else (t.data_ptr(), _lib.version_of(t)) for t in deps)
     hit = _DECODED.get(key)
     if hit is not None and hit[1] == versions and all(
             (r is None and t is None) or (r is not None and r() is t) for r, t in zip(hit[0], deps)):
         return hit[2]
-    if bounded and hit is None and not _decoded_fits(_nbytes(weight), weight.device):
+    if bounded and hit is None and not _decoded_fits(nbytes, weight.device):
         return None
-    dense = _mx_decoded(weight, code, scale, block_size, kdim)
+    dense = make()
     if torch.cuda.is_current_stream_capturing():
         return dense  # part of the graph being captured (its memory pool): decoded again on each replay
     # a later call may come on another stream: it finds the decode finished
@@ -975,6 +1005,13 @@ def _decoded_weight(weight, code, scale, block_size, kdim, bounded=False):
         weakref.finalize(weight, _release_decoded, key)
     _store_decoded(key, (tuple(None if t is None else weakref.ref(t) for t in deps), versions, dense))
     return dense
+
+
+def _decoded_weight(weight, code, scale, block_size, kdim, bounded=False):
+    """The bf16 decode of a convert-format weight in its own layout, cached
+    as the packed NF4 weight is."""
+    return _cached_decode(("dense", block_size, kdim), (weight, code, scale), _nbytes(weight),
+                          lambda: _mx_decoded(weight, code, scale, block_size, kdim), bounded)
 
 
 _DENSE_WS = {}
@@ -1037,26 +1074,56 @@ def _dense_weight_linear(a, a_code, a_scale, w, w_code, w_scale, block_size, bia
     return _dense_linear(_aligned16(a), _aligned16(w), None if bias is None else bias.contiguous())
 
 
-def _mx_product(a, a_code, a_scale, b, b_code, b_scale, block_size, b_stored_kn, bias, b_static=False):
-    """A'[*, M, K] . B' through vqx_mx_matmul, or None when the operands fall
-    outside it.  b: [*, K, N] when b_stored_kn, else [*, N, K]; batch dims
-    equal, or one side without them.  b_static: b is a weight (its decode is
-    cached when it is decoded ahead of the product)."""
-    if not (_mx_side_ok(a, a_code, a_scale, block_size, -1)
-            and _mx_side_ok(b, b_code, b_scale, block_size, -2 if b_stored_kn else -1)):
+def _dense_rows(t, code, scale, block_size, kdim, K):
+    """One operand of vqx_dense_matmul: [batch, rows, ceil(K / 64) * 64]
+    contiguous plain bf16 with K last, t itself where it already is that."""
+    if code is None and scale is None and K % 64 == 0:
+        r = t if kdim == -1 else t.transpose(-2, -1)
+        if r.is_contiguous() and r.data_ptr() % 16 == 0:
+            return r.reshape(-1, r.shape[-2], K)
+    return _mx_rows(t, code, scale, block_size, kdim, True, -(-K // 64) * 64)
+
+
+def _dense_product(a, a_code, a_scale, b, b_code, b_scale, block_size, b_kdim, bias, batch_shape, a_shared, b_shared):
+    """The product with both operands decoded ahead (each read by many output
+    tiles), any K, M and N; None past vqx_dense_matmul's 32-bit offsets."""
+    M, K = a.shape[-2], a.shape[-1]
+    N = b.shape[-2] if b_kdim == -1 else b.shape[-1]
+    batch = math.prod(batch_shape)
+    if b_shared and not a_shared:  # one right matrix for every item: the items' rows run as one product
+        rows, nb = batch * M, 1
+    else:
+        rows, nb = M, batch
+    Kp = -(-K // 64) * 64
+    if not _dense_takes(rows, N, Kp):
         return None
-    N = b.shape[-1] if b_stored_kn else b.shape[-2]
-    if (a_code is not None or a_scale is not None) and -(-N // 128) > _FUSED_DECODE_MAX_TILES:
-        a, a_code, a_scale = _mx_decoded(a, a_code, a_scale, block_size, -1), None, None
-    rows = a.shape[-2] * (math.prod(a.shape[:-2]) if b.dim() == 2 else 1)
-    if (b_code is not None or b_scale is not None) and -(-rows // 128) > _FUSED_DECODE_MAX_TILES:
-        kdim = -2 if b_stored_kn else -1
-        b = _decoded_weight(b, b_code, b_scale, block_size, kdim) if b_static else \
-            _mx_decoded(b, b_code, b_scale, block_size, kdim)
-        b_code, b_scale = None, None
+    ad = _dense_rows(a, a_code, a_scale, block_size, -1, K)
+    bd = _dense_rows(b, b_code, b_scale, block_size, b_kdim, K)
+    out = torch.empty(nb, rows, N, dtype=torch.bfloat16, device=a.device)
+    ws_bytes = _dense_workspace_bytes(nb, rows, N, Kp, a.device)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
+    _lib.call("vqx_dense_matmul", _lib.ptr(ad), Kp, 0 if a_shared or nb == 1 else rows * Kp, _lib.ptr(bd), Kp,
+              0 if b_shared else N * Kp, None if bias is None else _lib.ptr(bias.contiguous()), _lib.ptr(out), nb, rows,
+              N, Kp, _lib.ptr(ws), ws_bytes, _lib.stream_of(a))
+    return out.reshape(*batch_shape, M, N)
+
+
+def _mx_product(a, a_code, a_scale, b, b_code, b_scale, block_size, b_stored_kn, bias, b_static=False):
+    """A'[*, M, K] . B' on bf16 operands with scales along K, or None when the
+    operands fall outside it.  b: [*, K, N] when b_stored_kn, else [*, N, K];
+    batch dims equal, or one side without them.  b_static: b is a weight (its
+    decode is cached when it is decoded ahead of the product).
+
+    An operand that at most _FUSED_DECODE_MAX_TILES output tiles read is
+    decoded inside the product (vqx_mx_matmul); when neither is, or the
+    product's alignment rules refuse the shape, both are decoded ahead and the
+    dense product runs."""
+    bk = -2 if b_stored_kn else -1
+    if not (_mx_side_ok(a, a_code, a_scale, block_size, -1) and _mx_side_ok(b, b_code, b_scale, block_size, bk)):
+        return None
     M, K = a.shape[-2], a.shape[-1]
     Kb, N = (b.shape[-2], b.shape[-1]) if b_stored_kn else (b.shape[-1], b.shape[-2])
-    if Kb != K or M < 1 or N < 1 or K < 1 or K % 8 or N % 4:
+    if Kb != K or M < 1 or N < 1 or K < 1 or a.device != b.device:
         return None
     if bias is not None and (bias.dtype != torch.bfloat16 or tuple(bias.shape) != (N,) or bias.device != a.device):
         return None
@@ -1072,9 +1139,34 @@ def _mx_product(a, a_code, a_scale, b, b_code, b_scale, block_size, b_stored_kn,
     batch = math.prod(batch_shape)
     if batch < 1:
         return None
-    bd, bs_, bk_major, bld, _, _ = _right_operand(b, b_code, b_scale, block_size, b_stored_kn)
-    if not bk_major and N % 8:
+    a_inline = (a_code is not None or a_scale is not None) and -(-N // 128) <= _FUSED_DECODE_MAX_TILES
+    row_tiles = -(-(M * (batch if b_shared else 1)) // 128)
+    b_coded = b_code is not None or b_scale is not None
+    b_inline = b_coded and row_tiles <= _FUSED_DECODE_MAX_TILES
+    # the product kernel's own rules; a right operand decoded ahead may also
+    # be turned to K-major rows of any length
+    fits = K >= 8 and N % 4 == 0 and (K % 8 == 0 and (not b_stored_kn or N % 8 == 0))
+    turned = a_inline and b_coded and not b_inline and not fits and K >= 8 and N % 4 == 0
+    if not b_static and not turned and not (fits and (a_inline or b_inline)):
+        out = _dense_product(a, a_code, a_scale, b, b_code, b_scale, block_size, bk, bias, batch_shape, a_shared, b_shared)
+        if out is not None or not fits:
+            return out
+    if not fits and not turned:
         return None
+    if (a_code is not None or a_scale is not None) and not a_inline:
+        a, a_code, a_scale = _mx_decoded(a, a_code, a_scale, block_size, -1), None, None
+    if turned:
+        ld = -(-K // 8) * 8
+        bd, bs_, bk_major, bld = _mx_rows(b, b_code, b_scale, block_size, bk, True, ld), None, True, ld
+        b_code = None
+    else:
+        if b_coded and not b_inline:
+            b = _decoded_weight(b, b_code, b_scale, block_size, bk) if b_static else \
+                _mx_decoded(b, b_code, b_scale, block_size, bk)
+            b_code, b_scale = None, None
+        bd, bs_, bk_major, bld, _, _ = _right_operand(b, b_code, b_scale, block_size, b_stored_kn)
+        if not bk_major and N % 8:
+            return None
     nkb = 0 if a_scale is None else a_scale.shape[-1]
     if b_shared and not a_shared:
         # one right matrix for every item: the items' rows run as one product
@@ -1096,14 +1188,15 @@ def _mx_product(a, a_code, a_scale, b, b_code, b_scale, block_size, b_stored_kn,
     else:
         s_b = 0 if bs_ is None else bs_.shape[-2] * N
         s_ld = N
-    opb = _mx_operand(bd, bc, bs_, block_size, bk_major, 0 if b_shared else K * N, bld,
+    b_item = N * bld if bk_major else K * N
+    opb = _mx_operand(bd, bc, bs_, block_size, bk_major, 0 if b_shared else b_item, bld,
                       0 if (bs_ is None or b_shared) else s_b, s_ld)
     bias_c = None if bias is None else bias.contiguous()
     if bias_c is not None and bias_c.data_ptr() % 8:
         bias_c = bias_c.clone()
     out = torch.empty(nbatch, rows, N, dtype=torch.bfloat16, device=dev)
-    _lib.call("vqx_mx_matmul", _lib.ctypes.byref(opa), _lib.ctypes.byref(opb), _lib.ptr(bias_c), _lib.ptr(out),
-              nbatch, rows, N, K, _lib.stream_of(a))
+    _lib.call("vqx_mx_matmul_any" if turned else "vqx_mx_matmul", _lib.ctypes.byref(opa), _lib.ctypes.byref(opb),
+              _lib.ptr(bias_c), _lib.ptr(out), nbatch, rows, N, K, _lib.stream_of(a))
     return out.reshape(*batch_shape, M, N)
 
 
@@ -1159,7 +1252,7 @@ def linear_mx(input, weight, bias=None, *, input_scale=None, weight_scale=None, 
     if A_data is None:
         return dense
     return _spmm(A_data, A_indices, A_indptr, weight, weight_scale, weight_code, block_size, weight_layout,
-                 addend=dense)
+                 addend=dense, b_static=True)
 
 
 @_impl("matmul_mx")
@@ -1403,9 +1496,10 @@ def _scale_index(scale, shape, block_size):
 
 
 def _spmm(data, indices, indptr, B, B_scale=None, B_code=None, block_size=None, weight_layout="kc",
-          addend=None):
+          addend=None, b_static=False):
     """spmm_csr (quantized.py:816-878) on the GPU; with an addend of the
-    output's shape and dtype, addend + spmm in the same pass."""
+    output's shape and dtype, addend + spmm in the same pass.  b_static: B is
+    a weight (its decoded [K, N] form is cached)."""
     assert weight_layout in ("kc", "ck"), weight_layout
     _lib.require_device(B, "spmm_csr")
     if B.ndim < 2:
@@ -1430,10 +1524,13 @@ def _spmm(data, indices, indptr, B, B_scale=None, B_code=None, block_size=None, 
     if B.ndim > 2 and nbB != nb:
         raise ValueError(f"spmm_csr: B holds {nbB} matrices for {nb} CSR batches")
     K, N = (bc, br) if weight_layout == "kc" else (br, bc)
-    Bc = B.contiguous()
-    if B_code is None and B_scale is None and weight_layout == "ck":
-        Bt = Bc
-    else:
+    def decode():
+        Bc = B.contiguous()
+        if B_code is None and B_scale is None and weight_layout == "ck":
+            return Bc
+        if weight_layout == "kc" and out_dtype == torch.bfloat16 and nbB * K * N > 0 and B.ndim >= 2 and (
+                B_code is None or B_code.dtype == torch.bfloat16) and _mx_side_ok(Bc, B_code, B_scale, block_size, -1):
+            return _mx_rows(Bc, B_code, B_scale, block_size, -1, False)
         Bt = torch.empty((nbB, K, N), dtype=out_dtype, device=dev)
         code = None if B_code is None else B_code.reshape(-1).contiguous()
         scale = None if B_scale is None else B_scale.contiguous()
@@ -1447,13 +1544,23 @@ def _spmm(data, indices, indptr, B, B_scale=None, B_code=None, block_size=None, 
                   _lib.dtype_tag(code.dtype) if code is not None else 0, 0 if code is None else code.numel(),
                   _lib.ptr(scale), _lib.dtype_tag(scale.dtype) if scale is not None else 0, sb, sr, sc, rdiv, cdiv,
                   _lib.ptr(Bt), _lib.dtype_tag(out_dtype), _lib.stream_of(Bc))
+        return Bt
+
+    # a linear's weight is laid out once (78 us of a 512 x 4096 x 4096 outlier
+    # linear's 142 when done on every call), if it is not taken as it is
+    Bt = None
+    if b_static and B.ndim == 2 and not (B_code is None and B_scale is None and weight_layout == "ck"):
+        Bt = _cached_decode(("rows", weight_layout, block_size), (B, B_code, B_scale), K * N * out_dtype.itemsize, decode,
+                            bounded=True)
+    if Bt is None:
+        Bt = decode()
     out_shape = (*batch_shape, R, N)
     fuse = (addend is not None and addend.dtype == out_dtype and tuple(addend.shape) == out_shape
             and addend.is_contiguous() and addend.device == dev)
     out = torch.empty(out_shape, dtype=out_dtype, device=dev)
     _lib.call("vqx_spmm_csr", _lib.ptr(data2), dtag, _lib.ptr(indices2), _lib.ptr(indptr2), nb, R, data2.shape[1],
               _lib.ptr(Bt), _lib.dtype_tag(out_dtype), K * N if B.ndim > 2 else 0, K, N,
-              _lib.ptr(addend) if fuse else None, _lib.ptr(out), _lib.stream_of(Bc))
+              _lib.ptr(addend) if fuse else None, _lib.ptr(out), _lib.stream_of(B))
     if addend is not None and not fuse:
         return addend + out
     return out
