@@ -438,6 +438,21 @@ int vqx_mx_matmul_any(const VqxMxOperand* a, const VqxMxOperand* b, const uint16
                       int64_t batch, int64_t M, int64_t N, int64_t K, vqx_stream_t stream);
 
 /*
+ * The products of a decode step's attention (matmul_mx, src/vc/ops/
+ * quantized.py:371-421, with one to four left rows): contiguous operands
+ * a [batch][M][K] and b [batch][K][N], each with an optional code table (1 to
+ * 256 bf16 entries) and optional bf16 scales per block_size along K
+ * ([batch][M][ceil(K / block_size)], [batch][ceil(K / block_size)][N]),
+ * decoded as vqx_mx_matmul decodes them; out [batch][M][N] bf16, fp32
+ * accumulation.  M <= 4, M * K <= 16384; any K and N, any alignment;
+ * block_size a power of two >= 8.
+ */
+int vqx_mx_few_rows(const uint16_t* a, const uint16_t* a_scale, const uint16_t* a_code, int32_t a_code_len,
+                    const uint16_t* b, const uint16_t* b_scale, const uint16_t* b_code, int32_t b_code_len,
+                    int32_t block_size, uint16_t* out, int64_t batch, int64_t M, int64_t N, int64_t K,
+                    vqx_stream_t stream);
+
+/*
  * The product of two plain bf16 matrices with K contiguous, where
  * linear_mx / matmul_mx end once their operands are decoded (src/vc/ops/
  * quantized.py:328-333, 400-406): out[b][M][N] = a[b] . b[b]^T (+ bias), fp32

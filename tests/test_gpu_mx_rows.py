@@ -71,7 +71,9 @@ def test_operand_rows(vqx, R, C, kdim, coded, scaled):
 @pytest.mark.gpu
 @pytest.mark.parametrize("B,M,N,K", [((3,), 333, 333, 64), ((2, 2), 333, 128, 333), ((3,), 1300, 64, 77),
                                      ((2,), 5, 1999, 128), ((2,), 1, 128, 1999), ((3,), 700, 66, 130),
-                                     ((2,), 40, 33, 9), ((2,), 130, 4, 8), ((1,), 600, 1024, 200), ((2,), 3, 3, 3)])
+                                     ((2,), 40, 33, 9), ((2,), 130, 4, 8), ((1,), 600, 1024, 200), ((2,), 3, 3, 3),
+                                     ((2, 2), 4, 65, 513), ((3,), 2, 8, 512), ((1,), 1, 1, 1), ((2,), 4, 100, 4096),
+                                     ((2,), 4, 40, 4104), ((1,), 1, 70, 16384), ((2,), 1, 64, 1025)])
 @pytest.mark.parametrize("coded", [False, True])
 @pytest.mark.parametrize("form", ["plain", "b_shared", "a_shared", "kc", "b_transposed"])
 def test_odd_products(vqx, B, M, N, K, coded, form):

@@ -108,6 +108,7 @@ _SIGNATURES = {
     "vqx_nf4_linear_ws": ([_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _P, _I64, _P], ctypes.c_int),
     "vqx_mx_matmul": ([_P, _P, _P, _P, _I64, _I64, _I64, _I64, _P], ctypes.c_int),
     "vqx_mx_matmul_any": ([_P, _P, _P, _P, _I64, _I64, _I64, _I64, _P], ctypes.c_int),
+    "vqx_mx_few_rows": ([_P, _P, _P, _I32, _P, _P, _P, _I32, _I32, _P, _I64, _I64, _I64, _I64, _P], ctypes.c_int),
     "vqx_dense_matmul": ([_P, _I64, _I64, _P, _I64, _I64, _P, _P, _I64, _I64, _I64, _I64, _P, _I64, _P],
                          ctypes.c_int),
     "vqx_dense_matmul_workspace_size": ([_I64, _I64, _I64, _I64, ctypes.POINTER(_I64)], ctypes.c_int),

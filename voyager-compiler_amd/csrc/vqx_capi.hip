@@ -364,6 +364,19 @@ int vqx_mx_matmul_any(const VqxMxOperand* a, const VqxMxOperand* b, const uint16
                  N, K, true, (hipStream_t)stream);
 }
 
+int vqx_mx_few_rows(const uint16_t* a, const uint16_t* a_scale, const uint16_t* a_code, int32_t a_code_len,
+                    const uint16_t* b, const uint16_t* b_scale, const uint16_t* b_code, int32_t b_code_len,
+                    int32_t block_size, uint16_t* out, int64_t batch, int64_t M, int64_t N, int64_t K,
+                    vqx_stream_t stream) {
+  g_err[0] = 0;
+  if ((a_scale || b_scale) && (block_size < 8 || (block_size & (block_size - 1))))
+    return set_error(kErrInvalid, "mx_few_rows: block_size %d must be a power of two >= 8", (int)block_size);
+  const int64_t nkb = block_size > 0 ? (K + block_size - 1) / block_size : 0;
+  const MxOperand oa{a, a_scale, a_code, M * K, K, M * nkb, nkb, 1, block_size, a_code_len, 0};
+  const MxOperand ob{b, b_scale, b_code, K * N, N, nkb * N, N, 0, block_size, b_code_len, 0};
+  return mx_gemv(oa, ob, out, batch, M, N, K, (hipStream_t)stream);
+}
+
 int vqx_dense_matmul(const uint16_t* a, int64_t lda, int64_t a_batch_stride, const uint16_t* b, int64_t ldb,
                      int64_t b_batch_stride, const uint16_t* bias, uint16_t* out, int64_t batch, int64_t M,
                      int64_t N, int64_t K, void* workspace, int64_t workspace_bytes, vqx_stream_t stream) {

@@ -218,6 +218,8 @@ struct MxOperand {
 };
 int mx_gemm(const MxOperand& a, const MxOperand& b, const uint16_t* bias, uint16_t* out, int64_t batch, int64_t M,
             int64_t N, int64_t K, bool any, hipStream_t st);  // any: K-major operands of any K >= 8 and alignment
+int mx_gemv(const MxOperand& a, const MxOperand& b, uint16_t* out, int64_t batch, int64_t M, int64_t N, int64_t K,
+            hipStream_t st);
 int mx_decode(const MxOperand& x, int64_t batch, int64_t rows, int64_t K, uint16_t* out, int64_t out_ld, bool turn,
               hipStream_t st);
 

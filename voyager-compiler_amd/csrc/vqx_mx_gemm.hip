@@ -622,6 +622,156 @@ __global__ __launch_bounds__(256) void mx_turn_kernel(MxOpArgs o, uint16_t* __re
   }
 }
 
+// Products of few rows with an N-major right operand (a decode step's
+// attention: one query row against the K^T or V cache, [K][N] as quantize_mx
+// writes it), both decoded on the fly.  Bound by the one read of the right
+// operand and, per CU, by its decode (about 4 VALU per value): a workgroup of
+// 256 threads owns 8 LN columns of an item; its 256 / LN groups of LN lanes
+// each take a run of consecutive k rows, a lane 8 columns (one 16-byte load
+// per row, eight rows in flight; the scales are loaded when the block
+// changes).  LN = 8 reads whole 128-byte lines of a k row; LN = 2, for
+// products whose columns would leave CUs idle (P V: 128 columns an item),
+// spreads an item over more workgroups, placed on one XCD, whose L2 serves the
+// rest of each line.  The groups' fp32 sums are added across the lanes, then
+// the waves, in a fixed order; nothing is split over workgroups.
+// Measured, 32 x [1, 128] x [128, 1999] and 32 x [1, 1999] x [1999, 128]:
+// 10.5 + 11 us (16 MB each); turning the cache and running the dense product
+// took 21 + 27, one workgroup of 1024 threads per 64 columns 14.5 + 16.7.
+constexpr int kGemvA = 16384;  // decoded left values a workgroup can hold
+
+template <int CTRL>
+__device__ __forceinline__ float add_dpp(float v) {
+  return v + u2f((uint32_t)__builtin_amdgcn_update_dpp(0, (int)f2u(v), CTRL, 0xF, 0xF, false));
+}
+
+// Sum of v over the lanes that hold the same columns (lane % LN), everywhere.
+template <int LN>
+__device__ __forceinline__ float add_groups(float v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  v = add_dpp<0x128>(v);  // row_ror:8
+  if constexpr (LN == 2) {
+    v = add_dpp<0x124>(v);  // row_ror:4
+    v = add_dpp<0x4E>(v);   // quad_perm: lane ^ 2
+  }
+  auto s = __builtin_amdgcn_permlane16_swap(f2u(v), f2u(v), false, false);
+  v = u2f(s[0]) + u2f(s[1]);
+  s = __builtin_amdgcn_permlane32_swap(f2u(v), f2u(v), false, false);
+  v = u2f(s[0]) + u2f(s[1]);
+#endif
+  return v;
+}
+
+template <int DB, int MR, int LN>
+__global__ __launch_bounds__(256) void mx_gemv_kernel(MxOpArgs a, MxOpArgs b, uint16_t* __restrict__ out, int M, int N,
+                                                      int K, int tn, int batch) {
+  constexpr int kGroups = 256 / LN, kCols = 8 * LN;
+  __shared__ uint16_t tab[2 * kMaxCode + 2];
+  __shared__ uint16_t as[kGemvA];
+  __shared__ float part[MR][4][kCols];
+  // an item's tiles on one XCD (workgroups go to the eight in turn)
+  const int j8 = blockIdx.x >> 3;
+  const bool turn = (batch & 7) == 0;
+  const int64_t bi = turn ? (j8 / tn) * 8 + (blockIdx.x & 7) : blockIdx.x / tn;
+  const int n0 = (turn ? j8 % tn : blockIdx.x % tn) * kCols;
+
+  const int kg = threadIdx.x / LN, c = n0 + (threadIdx.x % LN) * 8, nv = N - c;
+  const int run = (K + kGroups - 1) / kGroups;
+  int k = kg * run;
+  const int kend = k + run < K ? k + run : K;
+  const uint16_t* bd = b.data + bi * b.bstride + c;
+  const uint16_t* sp = b.scale ? b.scale + bi * b.sbstride + c : nullptr;
+  u32x4 v[8];  // the first rows are under way while the left rows are decoded
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = k + i < kend ? load8(bd + (int64_t)(k + i) * b.ld, nv) : u32x4{0u, 0u, 0u, 0u};
+
+  u32x4 sc = {0u, 0u, 0u, 0u};
+  int blk = -1;
+  if constexpr (DB == kScale || DB == kCodeScale) {
+    if (k < kend) {
+      blk = k >> b.bs_shift;
+      sc = load8(sp + (int64_t)blk * b.sld, nv);
+    }
+  }
+
+  // the left rows, decoded as the reference's operand: bf16 values
+  const uint16_t* asc = a.scale ? a.scale + bi * a.sbstride : nullptr;
+  for (int m = 0; m < M; ++m)
+    for (int i = threadIdx.x * 8; i < K; i += 256 * 8) {
+      const u32x4 w = load8(a.data + bi * a.bstride + (int64_t)m * a.ld + i, K - i);
+      const float s = asc ? bf2f(asc[(int64_t)m * a.sld + (i >> a.bs_shift)]) : 1.0f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        if (i + e >= K) break;
+        float x = bf2f((w[e >> 1] >> (16 * (e & 1))) & 0xFFFFu);
+        if (a.code) {
+          const float t = __builtin_truncf(x);
+          const bool ok = t >= -(float)a.code_len && t < (float)a.code_len;
+          const int j = ok ? (int)t : 0;
+          x = ok ? bf2f(a.code[j < 0 ? j + a.code_len : j]) : __builtin_nanf("");
+        }
+        as[m * K + i + e] = (uint16_t)f2bf(x * s);  // without scales: x * 1
+      }
+    }
+  const int len = b.code_len;
+  if constexpr (DB >= kCode) {
+    for (int e = threadIdx.x; e < 2 * len + 2; e += 256) {
+      const int i = e - len - 1;
+      tab[e] = i >= -len && i < len ? b.code[i < 0 ? i + len : i] : (uint16_t)0x7FC0u;
+    }
+  }
+  __syncthreads();
+  const CodeLookup lk{tab, -(float)(len + 1), (float)len, len + 1};
+  float acc[MR][8];
+#pragma unroll
+  for (int m = 0; m < MR; ++m)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[m][e] = 0.0f;
+  while (k < kend) {
+    u32x4 nx[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      nx[i] = k + 8 + i < kend ? load8(bd + (int64_t)(k + 8 + i) * b.ld, nv) : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if (k + i >= kend) break;
+      if constexpr (DB == kScale || DB == kCodeScale) {
+        if (((k + i) >> b.bs_shift) != blk) {
+          blk = (k + i) >> b.bs_shift;
+          sc = load8(sp + (int64_t)blk * b.sld, nv);
+        }
+      }
+      float x[MR];
+#pragma unroll
+      for (int m = 0; m < MR; ++m) x[m] = m < M ? bf2f(as[m * K + k + i]) : 0.0f;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t d = decode_pair<DB>(v[i][j], bf_lo(sc[j]), bf_hi(sc[j]), lk);
+#pragma unroll
+        for (int m = 0; m < MR; ++m) {
+          acc[m][2 * j] += x[m] * bf_lo(d);
+          acc[m][2 * j + 1] += x[m] * bf_hi(d);
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = nx[i];
+    k += 8;
+  }
+#pragma unroll
+  for (int m = 0; m < MR; ++m)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float t = add_groups<LN>(acc[m][e]);
+      if ((threadIdx.x & 63) < LN) part[m][threadIdx.x >> 6][(threadIdx.x % LN) * 8 + e] = t;
+    }
+  __syncthreads();
+  for (int i = threadIdx.x; i < M * kCols; i += 256) {
+    const int m = i / kCols, col = i % kCols;
+    const float t = (part[m][0][col] + part[m][1][col]) + (part[m][2][col] + part[m][3][col]);
+    if (n0 + col < N) out[((int64_t)bi * M + m) * N + n0 + col] = (uint16_t)f2bf(t);
+  }
+}
+
 template <int DA, int DB, bool BK, int TM, int TN>
 int launch_one(const MxOpArgs& a, const MxOpArgs& b, const uint16_t* bias, uint16_t* out, int M, int N, int K,
                int batch, hipStream_t stream) {
@@ -817,6 +967,49 @@ int mx_decode(const MxOperand& x, int64_t batch, int64_t rows, int64_t K, uint16
     case kScale: return launch_decode<kScale>(km, o, out, iR, iC, il, (uint32_t)chunks, stream);
     case kCode: return launch_decode<kCode>(km, o, out, iR, iC, il, (uint32_t)chunks, stream);
     default: return launch_decode<kCodeScale>(km, o, out, iR, iC, il, (uint32_t)chunks, stream);
+  }
+}
+
+template <int DB, int MR>
+int launch_gemv(const MxOpArgs& a, const MxOpArgs& b, uint16_t* out, int64_t batch, int M, int N, int K,
+                hipStream_t stream) {
+  // whole lines of a k row when that gives every CU a workgroup
+  if (batch * ((N + 63) / 64) >= num_cus()) {
+    const int tn = (N + 63) / 64;
+    hipLaunchKernelGGL((mx_gemv_kernel<DB, MR, 8>), dim3((unsigned)(batch * tn)), dim3(256), 0, stream, a, b, out, M, N,
+                       K, tn, (int)batch);
+  } else {
+    const int tn = (N + 15) / 16;
+    hipLaunchKernelGGL((mx_gemv_kernel<DB, MR, 2>), dim3((unsigned)(batch * tn)), dim3(256), 0, stream, a, b, out, M, N,
+                       K, tn, (int)batch);
+  }
+  return check_launch("mx_gemv_kernel");
+}
+
+int mx_gemv(const MxOperand& a, const MxOperand& b, uint16_t* out, int64_t batch, int64_t M, int64_t N, int64_t K,
+            hipStream_t stream) {
+  if (batch < 1 || M < 1 || N < 1 || K < 1) return set_error(kErrInvalid, "mx_gemv: empty product");
+  if (M > 4 || M * K > kGemvA)
+    return set_error(kErrInvalid, "mx_gemv: at most 4 rows and %d left values", kGemvA);
+  if (b.k_major) return set_error(kErrInvalid, "mx_gemv: the right operand is N-major ([K][N])");
+  int rc = check_operand(a, "mx_gemv A", true, K, M, true);
+  if (rc) return rc;
+  rc = check_operand(b, "mx_gemv B", false, K, N, true);
+  if (rc) return rc;
+  if (!out || !aligned(out, 2)) return set_error(kErrInvalid, "mx_gemv: null or misaligned out");
+  if (N > INT32_MAX - 64 || batch * ((N + 15) / 16) > INT32_MAX)
+    return set_error(kErrInvalid, "mx_gemv: dimension too large");
+  const MxOpArgs aa = args_of(a), bb = args_of(b);
+  const int iM = (int)M, iN = (int)N, iK = (int)K;
+  switch (dec_of(b)) {
+#define VQX_GEMV(D)                                                                        \
+  return M == 1 ? launch_gemv<D, 1>(aa, bb, out, batch, iM, iN, iK, stream)                \
+                : launch_gemv<D, 4>(aa, bb, out, batch, iM, iN, iK, stream);
+    case kPlain: VQX_GEMV(kPlain)
+    case kScale: VQX_GEMV(kScale)
+    case kCode: VQX_GEMV(kCode)
+    default: VQX_GEMV(kCodeScale)
+#undef VQX_GEMV
   }
 }
 

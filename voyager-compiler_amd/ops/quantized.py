@@ -1255,6 +1255,46 @@ def linear_mx(input, weight, bias=None, *, input_scale=None, weight_scale=None, 
                  addend=dense, b_static=True)
 
 
+# The attention products of a decode step: up to four left rows against a
+# cache stored [K, N] read it once, in place (vqx_mx_few_rows).
+_FEW_ROWS, _FEW_ROWS_VALUES = 4, 16384
+
+
+def _few_rows_product(a, a_code, a_scale, b, b_code, b_scale, block_size):
+    """a[*, M, K] . b[*, K, N] with M <= 4 through vqx_mx_few_rows, or None
+    when the operands fall outside it."""
+    sa, sb = a.shape, b.shape
+    nd = len(sa)
+    if nd < 2 or nd != len(sb):
+        return None
+    M, K = sa[-2:]
+    N = sb[-1]
+    if not (0 < M <= _FEW_ROWS and 0 < K and M * K <= _FEW_ROWS_VALUES and N > 0 and sb[-2] == K and sa[:-2] == sb[:-2]):
+        return None
+    if not (_mx_side_ok(a, a_code, a_scale, block_size, -1) and _mx_side_ok(b, b_code, b_scale, block_size, -2)):
+        return None
+    dev = a.device
+    if b.device != dev or not (a.is_contiguous() and b.is_contiguous()):
+        return None
+    batch = math.prod(sa[:-2])
+    if batch < 1 or 2 * K * N >= 1 << 32:
+        return None
+    if a_scale is not None:
+        a_scale = a_scale.contiguous()
+    if b_scale is not None:
+        b_scale = b_scale.contiguous()
+    if a_code is not None:
+        a_code = _code_bf16(a_code, dev)
+    if b_code is not None:
+        b_code = _code_bf16(b_code, dev)
+    out = torch.empty((*sa[:-1], N), dtype=torch.bfloat16, device=dev)
+    _lib.call("vqx_mx_few_rows", a.data_ptr(), _lib.ptr(a_scale), _lib.ptr(a_code),
+              0 if a_code is None else a_code.numel(), b.data_ptr(), _lib.ptr(b_scale), _lib.ptr(b_code),
+              0 if b_code is None else b_code.numel(), block_size or 0, out.data_ptr(), batch, M, N, K,
+              _lib.stream_of(a))
+    return out
+
+
 @_impl("matmul_mx")
 def matmul_mx(self, other, *, input_scale=None, weight_scale=None, block_size=None, input_code=None,
               weight_code=None, A_data=None, A_indices=None, A_indptr=None, weight_layout="ck"):
@@ -1269,7 +1309,9 @@ def matmul_mx(self, other, *, input_scale=None, weight_scale=None, block_size=No
     transposed = weight_layout == "ck"
     dense = None
     a = None
-    if weight_code is not None and weight_code.numel() <= 16 and other.dim() == 2:
+    if transposed and other.dim() > 2 and _coded(input_code, input_scale, weight_code, weight_scale):
+        dense = _few_rows_product(self, input_code, input_scale, other, weight_code, weight_scale, block_size)
+    if dense is None and weight_code is not None and weight_code.numel() <= 16 and other.dim() == 2:
         a = _activation_decoded(self, input_code, input_scale, block_size)
         if a.dim() >= 1 and _fusable(a, other, None, weight_scale, block_size, weight_code, transposed):
             dense = _fused_linear(a, other, None, weight_scale, weight_code, transposed)
