@@ -1089,6 +1089,171 @@ __global__ __launch_bounds__(kMxLutThreads) void mx_lut_kernel(const uint16_t* _
   if constexpr (OUTL) outlier_tally(nskip, oa);
 }
 
+// The same stream for a table of all 65536 patterns (a qmap given as such: the
+// index table of a converted graph, a fitted codebook): the whole bf16 table,
+// 128 KiB, sits in LDS, one persistent workgroup of sixteen waves per CU, and
+// an element is its quotient's bf16 rounding and one 2-byte LDS read.  Reading
+// the table from the L2 instead bounds mx_group_kernel (2048 x 11008, nf4_6
+// index table: 34 us against 20, 4.5 TB/s); filling LDS costs about 3 us, so
+// inputs below kTableMin elements keep the gather (2^20 elements 4.6 us
+// against 4.9, 2^21 5.7 both, 2^22 8.6 against 6.3, 2^24 26.9 against 15.7).
+//
+// Quotients: power-of-two scales divide by an exact multiplication.  Absmax
+// scales multiply by v_rcp_f32, which rounds to the bf16 of the reference's
+// division as long as the quotient is normal (no quotient of bf16 values lies
+// within 2^-17 of a midpoint of normal bf16 values; a subnormal result can lie
+// on one, and its conversion is left to f2bf): a group whose smallest nonzero
+// magnitude divides to less than 2^-120, or whose scale or maximum is extreme,
+// NaN or Inf, divides exactly.
+constexpr int kTableMin = 1 << 21;
+
+template <int LPB, bool ABSMAX, int WANT>
+__global__ __launch_bounds__(kMxLutThreads) void mx_table_kernel(const uint16_t* __restrict__ x, int64_t ngroups,
+                                                                 ScaleParams sp, const uint16_t* __restrict__ table,
+                                                                 MxOut out) {
+  __shared__ __attribute__((aligned(16))) u32x4 tab[65536 / 8];
+  __shared__ uint8_t thr8[256];
+  const int lane = threadIdx.x & 63;
+  const int64_t nchunks = ngroups / 64;
+  const int64_t nwaves = (int64_t)gridDim.x * (blockDim.x / 64);
+  int64_t c = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6)));
+  const u32x4* xv = reinterpret_cast<const u32x4*>(x);
+  const uint32_t slot = half_slot(lane);
+  // the first chunk's loads are in flight while the table fills LDS
+  u32x4 n0 = {0, 0, 0, 0}, n1 = {0, 0, 0, 0};
+  if (c < nchunks) {
+    n0 = ld_nt(xv + c * 128 + slot);
+    n1 = ld_nt(xv + c * 128 + 64 + slot);
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    tab[i * kMxLutThreads + threadIdx.x] = reinterpret_cast<const u32x4*>(table)[i * kMxLutThreads + threadIdx.x];
+  if constexpr (!ABSMAX)
+    for (int i = threadIdx.x; i < 256; i += blockDim.x) thr8[i] = (uint8_t)log2_step_threshold(i);
+  __syncthreads();
+  const uint16_t* const t = reinterpret_cast<const uint16_t*>(tab);
+  const bool qmax_pow2 = (f2u(sp.quant_max) & 0x807FFFFFu) == 0 && ((f2u(sp.quant_max) >> 23) - 1u) < 253u;
+  const float qmax_rcp = u2f((254u - (f2u(sp.quant_max) >> 23)) << 23);
+
+  // one group of 16 consecutive elements (w, as bf16 pairs), index gl; SW: a
+  // whole chunk in the swapped layout
+  auto group = [&](auto sw, const uint32_t(&w)[8], int64_t gl) {
+    constexpr bool SW = decltype(sw)::value;
+    u16x2 m2 = {0, 0}, l2 = {0xFFFF, 0xFFFF};  // magnitude maxima, and minima less one (a zero wraps to the top)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const u16x2 mag = __builtin_bit_cast(u16x2, w[j] & 0x7FFF7FFFu);
+      m2 = __builtin_elementwise_max(m2, mag);
+      l2 = __builtin_elementwise_min(l2, (u16x2)(mag - (u16x2){1, 1}));
+    }
+    const uint32_t amax = block_max<LPB>((uint32_t)(m2.x > m2.y ? m2.x : m2.y));
+    float s;
+    if constexpr (ABSMAX) {
+      if (qmax_pow2 && !sp.scale_qmap) {
+        const float sc = u2f(pack_bf16x2(u2f(amax << 16) * qmax_rcp, 0.0f) << 16);
+        s = sc > 0.0f ? sc : 1.0f;
+      } else {
+        s = block_scale_bf16<true>(amax, sp);
+      }
+    } else {
+      s = block_scale_pow2_lds(amax, sp.shift, thr8);
+    }
+    const uint32_t sb = f2u(s), sE = (sb >> 23) & 0xFFu;
+    const uint32_t low = l2.x < l2.y ? l2.x : l2.y;  // 0xFFFF: all zeros
+    const float rcp = ABSMAX ? __builtin_amdgcn_rcpf(s) : u2f((254u - sE) << 23);
+    const bool fast = amax < 0x7F80u && sE >= 2 && sE <= 252 && (ABSMAX || (sb & 0x7FFFFFu) == 0) &&
+                      u2f(amax << 16) * rcp < 0x1p120f && (low == 0xFFFFu || u2f((low + 1u) << 16) * rcp >= 0x1p-120f);
+    uint32_t v[16];
+    if (fast) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint32_t hh = pack_bf16x2(u2f(w[j] << 16) * rcp, u2f(w[j] & 0xFFFF0000u) * rcp);
+        v[2 * j] = t[hh & 0xFFFFu];
+        v[2 * j + 1] = t[hh >> 16];
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const uint32_t xb = (j & 1) ? (w[j >> 1] & 0xFFFF0000u) : (w[j >> 1] << 16);
+        const float q = u2f(xb) / s;
+        const uint32_t h = f2bf(q);
+        v[j] = t[q == q ? h : (h & 0x7FFFu) | ((xb >> 16) & 0x8000u)];  // a NaN quotient takes x's sign
+      }
+    }
+    auto store = [&](uint16_t* base, const uint32_t(&b)[8]) {
+      if constexpr (SW) {
+        u32x4 a0 = {b[0], b[1], b[2], b[3]}, a1 = {b[4], b[5], b[6], b[7]};
+        half_swap(a0, a1);
+        u32x4* p = reinterpret_cast<u32x4*>(base + (gl - lane) * 16);
+        st_nt(p + slot, a0);
+        st_nt(p + 64 + slot, a1);
+      } else {
+        u32x4* p = reinterpret_cast<u32x4*>(base + gl * 16);
+        st_nt(p, u32x4{b[0], b[1], b[2], b[3]});
+        st_nt(p + 1, u32x4{b[4], b[5], b[6], b[7]});
+      }
+    };
+    if constexpr (WANT & 1) {
+      uint32_t b[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) b[j] = v[2 * j] | (v[2 * j + 1] << 16);
+      store(static_cast<uint16_t*>(out.qvals), b);
+    }
+    if constexpr (WANT & 2) {
+      uint32_t b[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        b[j] = f2bf(u2f(v[2 * j] << 16) * s) | (f2bf(u2f(v[2 * j + 1] << 16) * s) << 16);
+      store(static_cast<uint16_t*>(out.fq), b);
+    }
+    if ((gl & (LPB - 1)) == 0) {
+      const int64_t blk = gl / LPB;
+      if (out.scale) static_cast<uint16_t*>(out.scale)[blk] = (uint16_t)f2bf(s);
+      if (out.scale_f32) out.scale_f32[blk] = s;
+      if (out.scale_e8m0) out.scale_e8m0[blk] = (uint8_t)e8m0_of(s);
+    }
+  };
+  for (; c < nchunks; c += nwaves) {
+    u32x4 a = n0, b = n1;
+    if (c + nwaves < nchunks) {  // prefetch the next chunk
+      n0 = ld_nt(xv + (c + nwaves) * 128 + slot);
+      n1 = ld_nt(xv + (c + nwaves) * 128 + 64 + slot);
+    }
+    half_swap(a, b);
+    const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    group(std::true_type{}, w, c * 64 + lane);
+  }
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t g = nchunks * 64 + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < ngroups; g += stride) {
+    const u32x4 a = xv[2 * g], b = xv[2 * g + 1];
+    const uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    group(std::false_type{}, w, g);
+  }
+}
+
+template <int LPB, bool ABSMAX>
+static int launch_table_k(const uint16_t* x, int64_t ngroups, const ScaleParams& sp, const uint16_t* table,
+                          const MxOut& out, hipStream_t st) {
+  const int64_t need = (ngroups + kMxLutThreads - 1) / kMxLutThreads;
+  const dim3 grid((unsigned)(need < num_cus() ? need : num_cus())), block(kMxLutThreads);
+  const int want = (out.qvals ? 1 : 0) | (out.fq ? 2 : 0);
+  if (want == 1) hipLaunchKernelGGL((mx_table_kernel<LPB, ABSMAX, 1>), grid, block, 0, st, x, ngroups, sp, table, out);
+  else if (want == 2) hipLaunchKernelGGL((mx_table_kernel<LPB, ABSMAX, 2>), grid, block, 0, st, x, ngroups, sp, table, out);
+  else hipLaunchKernelGGL((mx_table_kernel<LPB, ABSMAX, 3>), grid, block, 0, st, x, ngroups, sp, table, out);
+  return check_launch("mx_quantize(table)");
+}
+
+template <bool ABSMAX>
+static int launch_table(const uint16_t* x, int64_t ngroups, int lpb, const ScaleParams& sp, const uint16_t* table,
+                        const MxOut& out, hipStream_t st) {
+  switch (lpb) {
+    case 1: return launch_table_k<1, ABSMAX>(x, ngroups, sp, table, out, st);
+    case 2: return launch_table_k<2, ABSMAX>(x, ngroups, sp, table, out, st);
+    case 4: return launch_table_k<4, ABSMAX>(x, ngroups, sp, table, out, st);
+    default: return launch_table_k<8, ABSMAX>(x, ngroups, sp, table, out, st);
+  }
+}
+
 template <int CB, int LPB, bool ABSMAX, int WANT>
 static int launch_lut_k(const uint16_t* x, int64_t ngroups, const ScaleParams& sp, const LutView& lv,
                         const MxOut& out, hipStream_t st) {
@@ -1520,6 +1685,14 @@ int mx_quantize(const void* x, int dtype, int64_t outer, int64_t L, int64_t inne
     if (fast) {
       LutView lv{fmt.lut, fmt.lut_len};
       return launch_lut((const uint16_t*)x, n, (int)lpb, packed ? fmt.code_bits : 0, sp, lv, out, st);
+    }
+    if (dtype == kBF16 && fmt.kind == kFmtTable && fmt.value_table && aligned(fmt.value_table, 16) && inner == 1 &&
+        bs % 16 == 0 && L % bs == 0 && lpb >= 1 && lpb <= 8 && (lpb & (lpb - 1)) == 0 && aligned(x, 16) &&
+        (!out.qvals || aligned(out.qvals, 16)) && (!out.fq || aligned(out.fq, 16)) && !out.codes &&
+        (out.qvals || out.fq) && !oa.active && n >= kTableMin) {
+      const int64_t ng = n / 16;
+      return sp.mode == 1 ? launch_table<true>((const uint16_t*)x, ng, (int)lpb, sp, fmt.value_table, out, st)
+                          : launch_table<false>((const uint16_t*)x, ng, (int)lpb, sp, fmt.value_table, out, st);
     }
     // blocks along a middle axis of a bf16 input: the table-driven column kernel
     const bool cols = dtype == kBF16 && fmt.lut && inner > 1 && inner % 8 == 0 && bs <= 16 * kColRowsMax &&
