@@ -431,8 +431,9 @@ int vqx_mx_matmul(const VqxMxOperand* a, const VqxMxOperand* b, const uint16_t* 
                   int64_t batch, int64_t M, int64_t N, int64_t K, vqx_stream_t stream);
 
 /*
- * vqx_mx_matmul on K-major operands (b.k_major = 1) of any K >= 8, alignment
- * and strides: a 2-byte aligned row is read in 16-byte loads all the same.
+ * vqx_mx_matmul on K-major operands (b.k_major = 1, already plain bf16: no
+ * code, no scale) of any K >= 8, alignment and strides: a 2-byte aligned row
+ * is read in 16-byte loads all the same.
  */
 int vqx_mx_matmul_any(const VqxMxOperand* a, const VqxMxOperand* b, const uint16_t* bias, uint16_t* out,
                       int64_t batch, int64_t M, int64_t N, int64_t K, vqx_stream_t stream);

@@ -149,9 +149,10 @@ __device__ __forceinline__ uint32_t valid_mask(int n, int j) {
 // Loads are never skipped (a branch around a load makes the compiler wait for
 // every load in flight at the join): past the last row the last row is read,
 // past K the last 8 values, and in a checked step the values past K are zeroed
-// after the decode.  K and the row stride may be any (K >= 8).  Addresses are a uniform base (the batch item) plus 32-bit byte
+// after the decode.  ANY: K and the row stride may be any (K >= 8), else both
+// are multiples of 8 and rows 16-byte aligned.  Addresses are a uniform base (the batch item) plus 32-bit byte
 // offsets; LDS addresses are precomputed.
-template <int D, int ROWS, int THREADS>
+template <int D, int ROWS, int THREADS, bool ANY>
 struct KMajor {
   static constexpr int kCh = ROWS * 8 / THREADS;  // chunks per thread
   static_assert(kCh >= 1 && kCh <= 4, "chunks per thread");
@@ -182,14 +183,15 @@ struct KMajor {
     int kl = k;
     x.in = 8;
     if constexpr (CHECK) {
-      x.in = K - k;  // 8 or more: all
+      x.in = K - k;  // 8 or more: all; K % 8 == 0 without ANY: all or none
       kl = k < K - 8 ? k : K - 8;
     }
     const uint32_t kb = 2u * (uint32_t)(kl - (int)(threadIdx.x & 7) * 8);
-    const int ksc = CHECK && k >= K ? kl : k;  // a chunk wholly past K takes any scale
+    const int ksc = ANY && CHECK && k < K ? k : kl;  // a chunk wholly past K takes any scale
 #pragma unroll
     for (int q = 0; q < kCh; ++q) {
-      x.v[q] = load16_any(base + (off[q] + kb));
+      if constexpr (ANY) x.v[q] = load16_any(base + (off[q] + kb));
+      else x.v[q] = *reinterpret_cast<const u32x4*>(base + (off[q] + kb));
       if constexpr (D == kScale || D == kCodeScale)
         x.s[q] = *reinterpret_cast<const uint16_t*>(sbase + (soff[q] + 2u * (uint32_t)(ksc >> sh)));
     }
@@ -202,13 +204,13 @@ struct KMajor {
     for (int q = 0; q < kCh; ++q) {
       const float s = bf_lo(x.s[q]);
       u32x4 d, v = x.v[q];
-      if constexpr (CHECK) {
+      if constexpr (ANY && CHECK) {
         if (x.in < 8) v = shift_down(v, (8 - x.in) & 7);  // loaded from K - 8 on
       }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         d[j] = decode2<D>(v[j], s, s, tab);
-        if constexpr (CHECK) d[j] &= valid_mask(x.in, j);
+        if constexpr (CHECK) d[j] = ANY ? d[j] & valid_mask(x.in, j) : (x.in > 0 ? d[j] : 0u);
       }
       *reinterpret_cast<u32x4*>(stage + lds[q]) = d;
     }
@@ -359,7 +361,7 @@ struct Shape {
   static constexpr int kStageA = TM * kTK * 2, kStageB = TN * kTK * 2;
 };
 
-template <int DA, int DB, bool BK, int TM, int TN>
+template <int DA, int DB, bool BK, int TM, int TN, bool ANY>
 __global__ __launch_bounds__((TM == 128 && TN == 128) ? 256 : 512, 2) void mx_gemm_kernel(
     MxOpArgs a, MxOpArgs b, const uint16_t* __restrict__ bias, uint16_t* __restrict__ out, int M, int N, int K, int tm,
     int tn, int ntiles) {
@@ -384,9 +386,9 @@ __global__ __launch_bounds__((TM == 128 && TN == 128) ? 256 : 512, 2) void mx_ge
   if constexpr (DB >= kCode) build_code_table<kThreads>(tb, b.code, b.code_len);
   if constexpr (DA >= kCode || DB >= kCode) __syncthreads();
 
-  KMajor<DA, TM, kThreads> sa;
+  KMajor<DA, TM, kThreads, ANY> sa;
   sa.init(a, bi, m0, M);
-  typename std::conditional<BK, KMajor<DB, TN, kThreads>, NMajor<DB, TN, kThreads>>::type sb;
+  typename std::conditional<BK, KMajor<DB, TN, kThreads, ANY>, NMajor<DB, TN, kThreads>>::type sb;
   sb.init(b, bi, n0, N);
 
   const int nk = (K + kTK - 1) / kTK;
@@ -515,6 +517,8 @@ __device__ __forceinline__ uint32_t decode_pair(uint32_t w, float s0, float s1, 
   }
 }
 
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(2)));
+
 // Up to n values from p, zeros behind them.
 __device__ __forceinline__ u32x4 load8(const uint16_t* p, int n) {
   if (n >= 8) return load16_any(reinterpret_cast<const char*>(p));
@@ -529,8 +533,11 @@ __device__ __forceinline__ u32x4 load8(const uint16_t* p, int n) {
 // stride o.ld, any alignment), out is [items][R][CP] contiguous with CP >= C
 // a multiple of 8, zeros past C; KMAJ: C = K, blocks along C; else R = K,
 // blocks along R.  Each thread decodes 8 consecutive values of a row per
-// iteration.
-template <int D, bool KMAJ>
+// iteration.  NT: non-temporal loads and stores, for the product that decodes
+// its other operand itself (P V of 2048 tokens 92 -> 85 us: P streams past
+// the decoded V); the dense product finds plainly stored operands in the
+// caches (scores of 2048 tokens 110 -> 90 us, 1000 x 4096 x 4096 41 -> 35).
+template <int D, bool KMAJ, bool NT>
 __global__ __launch_bounds__(256) void mx_decode_kernel(MxOpArgs o, uint16_t* __restrict__ out, int R, int C, int CP,
                                                         uint32_t chunks) {
   __shared__ uint16_t tab[D >= kCode ? 2 * kMaxCode + 2 : 1];
@@ -544,7 +551,9 @@ __global__ __launch_bounds__(256) void mx_decode_kernel(MxOpArgs o, uint16_t* __
     const int n = C - c;  // values of the chunk inside the row
     u32x4 d = {0u, 0u, 0u, 0u};
     if (n > 0) {
-      const u32x4 v = load8(o.data + (int64_t)bi * o.bstride + (int64_t)r * o.ld + c, n);
+      const uint16_t* src = o.data + (int64_t)bi * o.bstride + (int64_t)r * o.ld + c;
+      const u32x4 v =
+          NT && n >= 8 ? __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(src)) : load8(src, n);
       u32x4 sc = {0u, 0u, 0u, 0u};
       float s = 1.0f;
       if constexpr (D == kScale || D == kCodeScale) {
@@ -556,7 +565,9 @@ __global__ __launch_bounds__(256) void mx_decode_kernel(MxOpArgs o, uint16_t* __
       for (int j = 0; j < 4; ++j)
         d[j] = decode_pair<D>(v[j], KMAJ ? s : bf_lo(sc[j]), KMAJ ? s : bf_hi(sc[j]), lk) & valid_mask(n, j);
     }
-    *reinterpret_cast<u32x4*>(out + (int64_t)row * CP + c) = d;
+    u32x4* const dst = reinterpret_cast<u32x4*>(out + (int64_t)row * CP + c);
+    if constexpr (NT) st_nt(dst, d);
+    else *dst = d;
   }
 }
 
@@ -772,13 +783,13 @@ __global__ __launch_bounds__(256) void mx_gemv_kernel(MxOpArgs a, MxOpArgs b, ui
   }
 }
 
-template <int DA, int DB, bool BK, int TM, int TN>
+template <int DA, int DB, bool BK, int TM, int TN, bool ANY = false>
 int launch_one(const MxOpArgs& a, const MxOpArgs& b, const uint16_t* bias, uint16_t* out, int M, int N, int K,
                int batch, hipStream_t stream) {
   const int tm = (M + TM - 1) / TM, tn = (N + TN - 1) / TN;
   const int64_t ntiles = (int64_t)batch * tm * tn;
   if (ntiles > INT32_MAX) return set_error(kErrInvalid, "mx_gemm: too many tiles");
-  hipLaunchKernelGGL((mx_gemm_kernel<DA, DB, BK, TM, TN>), dim3((unsigned)ntiles), dim3(Shape<TM, TN>::kThreads), 0,
+  hipLaunchKernelGGL((mx_gemm_kernel<DA, DB, BK, TM, TN, ANY>), dim3((unsigned)ntiles), dim3(Shape<TM, TN>::kThreads), 0,
                      stream, a, b, bias, out, M, N, K, tm, tn, (int)ntiles);
   return check_launch("mx_gemm_kernel");
 }
@@ -903,6 +914,15 @@ int mx_gemm(const MxOperand& a, const MxOperand& b, const uint16_t* bias, uint16
                       b.ld, b.batch_stride, bias, out, batch, M, N, K, nullptr, 0, stream);
   const MxOpArgs aa = args_of(a), bb = args_of(b);
   const int db = dec_of(b);
+  if (any) {
+    if (db != kPlain) return set_error(kErrInvalid, "mx_gemm: a plain right operand needed for operands of any K");
+    switch (dec_of(a)) {
+      case kPlain: return launch_one<kPlain, kPlain, true, 128, 128, true>(aa, bb, bias, out, (int)M, (int)N, (int)K, (int)batch, stream);
+      case kScale: return launch_one<kScale, kPlain, true, 128, 128, true>(aa, bb, bias, out, (int)M, (int)N, (int)K, (int)batch, stream);
+      case kCode: return launch_one<kCode, kPlain, true, 128, 128, true>(aa, bb, bias, out, (int)M, (int)N, (int)K, (int)batch, stream);
+      default: return launch_one<kCodeScale, kPlain, true, 128, 128, true>(aa, bb, bias, out, (int)M, (int)N, (int)K, (int)batch, stream);
+    }
+  }
   const bool bk = b.k_major != 0;
   const int tile = pick_tile(batch, M, N, K);
   const int iM = (int)M, iN = (int)N, iK = (int)K, ib = (int)batch;
@@ -914,15 +934,20 @@ int mx_gemm(const MxOperand& a, const MxOperand& b, const uint16_t* bias, uint16
   }
 }
 
-template <int D>
-int launch_decode(bool kmaj, const MxOpArgs& o, uint16_t* out, int R, int C, int CP, uint32_t chunks,
-                  hipStream_t stream) {
-  const unsigned grid = grid_for(chunks, 256, 8);
-  if (kmaj)
-    hipLaunchKernelGGL((mx_decode_kernel<D, true>), dim3(grid), dim3(256), 0, stream, o, out, R, C, CP, chunks);
-  else
-    hipLaunchKernelGGL((mx_decode_kernel<D, false>), dim3(grid), dim3(256), 0, stream, o, out, R, C, CP, chunks);
+template <int D, bool NT>
+int launch_decode_nt(bool kmaj, const MxOpArgs& o, uint16_t* out, int R, int C, int CP, uint32_t chunks,
+                     hipStream_t stream) {
+  const dim3 grid(grid_for(chunks, 256, 8)), block(256);
+  if (kmaj) hipLaunchKernelGGL((mx_decode_kernel<D, true, NT>), grid, block, 0, stream, o, out, R, C, CP, chunks);
+  else hipLaunchKernelGGL((mx_decode_kernel<D, false, NT>), grid, block, 0, stream, o, out, R, C, CP, chunks);
   return check_launch("mx_decode_kernel");
+}
+
+template <int D>
+int launch_decode(bool kmaj, bool nt, const MxOpArgs& o, uint16_t* out, int R, int C, int CP, uint32_t chunks,
+                  hipStream_t stream) {
+  return nt ? launch_decode_nt<D, true>(kmaj, o, out, R, C, CP, chunks, stream)
+            : launch_decode_nt<D, false>(kmaj, o, out, R, C, CP, chunks, stream);
 }
 
 template <int D>
@@ -937,7 +962,7 @@ int launch_turn(bool srow, const MxOpArgs& o, uint16_t* out, int R, int C, int R
 // x decoded into dense bf16: in its own layout (turn 0, rows padded with zeros
 // to out_ld, a multiple of 8), or with its two dims swapped (turn 1).
 int mx_decode(const MxOperand& x, int64_t batch, int64_t rows, int64_t K, uint16_t* out, int64_t out_ld, bool turn,
-              hipStream_t stream) {
+              bool nt, hipStream_t stream) {
   if (batch < 1 || rows < 1 || K < 1) return set_error(kErrInvalid, "mx_decode: empty operand");
   int rc = check_operand(x, "mx_decode", false, K, rows, true);
   if (rc) return rc;
@@ -963,10 +988,10 @@ int mx_decode(const MxOperand& x, int64_t batch, int64_t rows, int64_t K, uint16
   const int64_t chunks = batch * R * (out_ld / 8);
   if (chunks > INT32_MAX) return set_error(kErrInvalid, "mx_decode: operand too large");
   switch (d) {
-    case kPlain: return launch_decode<kPlain>(km, o, out, iR, iC, il, (uint32_t)chunks, stream);
-    case kScale: return launch_decode<kScale>(km, o, out, iR, iC, il, (uint32_t)chunks, stream);
-    case kCode: return launch_decode<kCode>(km, o, out, iR, iC, il, (uint32_t)chunks, stream);
-    default: return launch_decode<kCodeScale>(km, o, out, iR, iC, il, (uint32_t)chunks, stream);
+    case kPlain: return launch_decode<kPlain>(km, nt, o, out, iR, iC, il, (uint32_t)chunks, stream);
+    case kScale: return launch_decode<kScale>(km, nt, o, out, iR, iC, il, (uint32_t)chunks, stream);
+    case kCode: return launch_decode<kCode>(km, nt, o, out, iR, iC, il, (uint32_t)chunks, stream);
+    default: return launch_decode<kCodeScale>(km, nt, o, out, iR, iC, il, (uint32_t)chunks, stream);
   }
 }
 

@@ -13,6 +13,7 @@ Ops beyond the reference's (packed storage is this build's own):
 """
 
 import ctypes
+import functools
 import math
 import threading
 import weakref
@@ -784,6 +785,8 @@ def _code_bf16(code: torch.Tensor, device) -> torch.Tensor:
     """The code table as the bf16 values the kernel reads (the reference casts
     the looked-up values to the operand's dtype, bf16 here), cached per code
     tensor and version."""
+    if code.dtype == torch.bfloat16 and code.device == device and code.is_contiguous():
+        return code
     key = (code.data_ptr(), _lib.version_of(code), code.numel(), code.dtype, str(device))
     hit = _BF16_CODES.get(key)
     if hit is not None and hit[0]() is code:
@@ -804,9 +807,10 @@ def _mx_side_ok(t, code, scale, block_size, kdim):
     if scale is not None:
         if block_size is None or block_size < 8 or block_size & (block_size - 1) or scale.dtype != torch.bfloat16:
             return False
-        want = list(t.shape)
-        want[kdim] = -(-want[kdim] // block_size)
-        if list(scale.shape) != want or scale.device != t.device:
+        ts, ss = t.shape, scale.shape
+        other = -1 if kdim == -2 else -2
+        if len(ts) != len(ss) or ss[kdim] != -(-ts[kdim] // block_size) or ss[other] != ts[other] \
+                or ss[:-2] != ts[:-2] or scale.device != t.device:
             return False
     return True
 
@@ -814,7 +818,10 @@ def _mx_side_ok(t, code, scale, block_size, kdim):
 def _coded(*parts):
     """Whether any operand carries a code table or scales (a product of two
     plain bf16 operands is the library GEMM's)."""
-    return any(p is not None for p in parts)
+    for p in parts:
+        if p is not None:
+            return True
+    return False
 
 
 def _aligned16(t):
@@ -823,16 +830,12 @@ def _aligned16(t):
 
 
 def _mx_operand(data, code, scale, block_size, k_major, batch_stride, ld, scale_batch_stride, scale_ld):
-    op = _lib.VqxMxOperand()
-    op.data = data.data_ptr()
-    op.scale = None if scale is None else scale.data_ptr()
-    op.code = None if code is None else code.data_ptr()
-    op.batch_stride, op.ld = batch_stride, ld
-    op.scale_batch_stride, op.scale_ld = scale_batch_stride, scale_ld
-    op.k_major = 1 if k_major else 0
-    op.block_size = 0 if scale is None else int(block_size)
-    op.code_len = 0 if code is None else code.numel()
-    return op
+    # positional, in the structure's field order: one call instead of a
+    # descriptor write per field
+    return _lib.VqxMxOperand(data.data_ptr(), None if scale is None else scale.data_ptr(),
+                             None if code is None else code.data_ptr(), batch_stride, ld, scale_batch_stride, scale_ld,
+                             1 if k_major else 0, 0 if scale is None else int(block_size),
+                             0 if code is None else code.numel(), 0)
 
 
 def _right_operand(b, code, scale, block_size, stored_kn):
@@ -943,21 +946,18 @@ def _mx_rows(t, code, scale, block_size, kdim, k_last=True, ld=None):
     dense bf16 rows of K (k_last) padded with zeros to ld, or rows of the
     other dim, turned on the way when t is stored in the other order
     (vqx_mx_operand_rows): [batch, rows, ld], batch dims flattened."""
-    lead = t.shape[:-2]
-    tt = t.transpose(-2, -1)
     if t.is_contiguous():
         m, flipped = t, False
-    elif tt.is_contiguous():
-        m, flipped = tt, True
     else:
-        m, flipped = t.contiguous(), False
+        tt = t.transpose(-2, -1)
+        m, flipped = (tt, True) if tt.is_contiguous() else (t.contiguous(), False)
     k_major = (kdim == -1) != flipped
     R, C = m.shape[-2], m.shape[-1]
     K, cols = (C, R) if k_major else (R, C)
     sm = None
     if scale is not None:
         sm = (scale.transpose(-2, -1) if flipped else scale).contiguous()
-    batch = math.prod(lead)
+    batch = math.prod(t.shape[:-2])
     op = _mx_operand(m, None if code is None else _code_bf16(code, t.device), sm, block_size, k_major, R * C, C,
                      0 if sm is None else sm.shape[-2] * sm.shape[-1], 0 if sm is None else sm.shape[-1])
     last, outer = (K, cols) if k_last else (cols, K)
@@ -1070,7 +1070,7 @@ def _dense_weight_linear(a, a_code, a_scale, w, w_code, w_scale, block_size, bia
         if w is None:
             return None
     if a_code is not None or a_scale is not None:
-        a = _mx_decoded(a, a_code, a_scale, block_size, -1)
+        a = _mx_rows(a, a_code, a_scale, block_size, -1)[0]
     return _dense_linear(_aligned16(a), _aligned16(w), None if bias is None else bias.contiguous())
 
 
@@ -1385,8 +1385,7 @@ def _outlier_csr(input, threshold, max_pct, indptr_offset):
         raise ValueError(f"filter_outlier: max_pct {max_pct} gives a negative capacity")
     if not -(1 << 31) <= indptr_offset < (1 << 31):
         raise ValueError(f"indptr_offset {indptr_offset} does not fit the int32 row pointers")
-    # torch compares against the Python scalar cast to the tensor's dtype
-    t = torch.tensor(float(threshold), dtype=x.dtype).item()
+    t = _threshold_in(float(threshold), x.dtype)
     nb = math.prod(batch_shape)
     dev = x.device
     data = torch.empty((*batch_shape, max_nnz), dtype=x.dtype, device=dev)
@@ -1399,12 +1398,23 @@ def _outlier_csr(input, threshold, max_pct, indptr_offset):
     return data, indices, indptr, inlier
 
 
+@functools.lru_cache(maxsize=1024)
+def _threshold_in(threshold, dtype):
+    """A Python threshold as torch compares it: cast to the tensor's dtype."""
+    return torch.tensor(threshold, dtype=dtype).item()
+
+
+@functools.lru_cache(maxsize=1024)
+def _outlier_workspace_bytes(tag, nb, R, C, max_nnz):
+    n = ctypes.c_int64(0)
+    _lib.call("vqx_outlier_workspace_size", tag, nb, R, C, max_nnz, ctypes.byref(n))
+    return max(n.value, 1)
+
+
 def _outlier_workspace(tag, nb, R, C, max_nnz, dev):
     """Staging memory of the one-pass outlier split: each row's count and its
     first outliers (the library sizes it; the caching allocator keeps it)."""
-    n = ctypes.c_int64(0)
-    _lib.call("vqx_outlier_workspace_size", tag, nb, R, C, max_nnz, ctypes.byref(n))
-    return torch.empty(max(n.value, 1), dtype=torch.uint8, device=dev)
+    return torch.empty(_outlier_workspace_bytes(tag, nb, R, C, max_nnz), dtype=torch.uint8, device=dev)
 
 
 @_impl("filter_outlier")
@@ -1445,7 +1455,7 @@ def _quantize_mx_outlier_fused(input, qmap, block_size, quant_max, force_pow2, s
         raise ValueError(f"filter_outlier: max_pct {max_pct} gives a negative capacity")
     if not -(1 << 31) <= indptr_offset < (1 << 31):
         raise ValueError(f"indptr_offset {indptr_offset} does not fit the int32 row pointers")
-    t = torch.tensor(float(threshold), dtype=x.dtype).item()
+    t = _threshold_in(float(threshold), x.dtype)
     nb = math.prod(batch_shape)
     dev = x.device
     data = torch.empty((*batch_shape, max_nnz), dtype=x.dtype, device=dev)
