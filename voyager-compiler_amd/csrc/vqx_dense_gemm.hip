@@ -27,8 +27,8 @@
 // What bounds kWide (2048 x 11008 x 4096, 688 tiles = 2.69 rounds of the
 // CUs): per step and CU 1024 cycles of MFMA against 1152 of LDS (96 KiB of
 // fragment reads, 48 KiB of fills, 128 B per cycle) and 768 of the vector
-// memory path; by counters (2048 x 4096 x 11008) the MFMA pipe is busy 73% of
-// the cycles, at the 1.6 GHz the power limit leaves.  A 256 x 256 tile of 8
+// memory path; by counters (2048 x 4096 x 11008) the MFMA pipe is busy 77% of
+// the cycles, at the 1.6 GHz the power limit leaves (141 us).  A 256 x 256 tile of 8
 // waves reads less LDS per product and keeps the pipe 85% busy at 8192^3, but
 // at 1.4 GHz, and leaves 1.34 rounds here: 166 to 184 us.
 //
