@@ -876,7 +876,10 @@ _DECODED = {}
 # back with the weight.
 _DECODED_SHARE = 4
 _DECODED_BYTES = {}
-_DECODED_LOCK = threading.Lock()
+# Reentrant, and the total is updated with no allocation between its read and
+# its write: a garbage collection inside the update can end another weight,
+# whose finalizer drops its entry from the same thread.
+_DECODED_LOCK = threading.RLock()
 _DEVICE_BYTES = {}
 
 
@@ -890,8 +893,8 @@ def _store_decoded(key, entry):
         old = _DECODED.pop(key, None)
         for e, sign in ((old, -1), (entry, 1)):
             if e is not None:
-                d = e[2].device.index
-                _DECODED_BYTES[d] = _DECODED_BYTES.get(d, 0) + sign * _nbytes(e[2])
+                d, n = e[2].device.index, sign * _nbytes(e[2])
+                _DECODED_BYTES[d] = _DECODED_BYTES.get(d, 0) + n
         if entry is not None:
             _DECODED[key] = entry
 
