@@ -996,6 +996,10 @@ def _cached_decode(form, deps, nbytes, make, bounded):
     hit = _DECODED.get(key)
     if hit is not None and hit[1] == versions and all(
             (r is None and t is None) or (r is not None and r() is t) for r, t in zip(hit[0], deps)):
+        if _lib.stream_of(weight) != hit[3]:
+            # allocated on another stream: its memory is not reused before
+            # the work queued here has read it, even if the weight goes first
+            hit[2].record_stream(torch.cuda.current_stream(weight.device))
         return hit[2]
     if bounded and hit is None and not _decoded_fits(nbytes, weight.device):
         return None
@@ -1006,7 +1010,8 @@ def _cached_decode(form, deps, nbytes, make, bounded):
     torch.cuda.current_stream(weight.device).synchronize()
     if hit is None:
         weakref.finalize(weight, _release_decoded, key)
-    _store_decoded(key, (tuple(None if t is None else weakref.ref(t) for t in deps), versions, dense))
+    _store_decoded(key, (tuple(None if t is None else weakref.ref(t) for t in deps), versions, dense,
+                         _lib.stream_of(weight)))
     return dense
 
 
