@@ -550,9 +550,9 @@ def setup_c6_mxnf4_linear(vqx, torch, L, M=2048, N=11008, K=4096):
     """The MXNF4 CI scheme's linear at the LLaMA-7B MLP shape through
     quantized_ops::linear_mx: nf4_6 activation indices with input_code and
     fp8_e5m3-grid input_scale per 64 along K, a convert-format nf4_6 weight
-    (16-entry weight_code, weight_scale per 64): the activation's decode pass,
-    then the dense product (graph replay of one call; the weight is decoded
-    once, cached)."""
+    (16-entry weight_code, weight_scale per 64): graph replay of one call, i.e.
+    the decode passes of both operands (a captured call decodes the weight in
+    the graph), then the dense product."""
     g = torch.Generator().manual_seed(8)
     bs = 64
     code = torch.tensor([-31., -22., -16., -12., -9., -6., -3., 0., 2., 5., 8., 10., 14., 17., 22., 31.],
@@ -575,8 +575,8 @@ def setup_c6_mxint8_linear(vqx, torch, L, M=2048, N=11008, K=4096):
     """The MXINT8 CI scheme's linear at the LLaMA-7B MLP shape through
     quantized_ops::linear_mx: int8 activations and weights (integer-valued
     bf16, as convert writes them), power-of-two bf16 scales per 16 along K on
-    both sides (graph replay of one call: the activation's decode, the
-    product; the weight's decode is cached per weight)."""
+    both sides (graph replay of one call: the decode passes of both operands,
+    as a captured call decodes the weight in the graph, then the product)."""
     g = torch.Generator().manual_seed(7)
     bs = 16
     x = torch.randint(-127, 128, (M, K), generator=g).to(torch.bfloat16).cuda()

@@ -1,5 +1,6 @@
-"""The cache of decoded weights: entries dropped while it is being changed, and
-entries used on another stream than the one they were made on."""
+"""The cache of decoded weights: entries dropped while it is being changed,
+entries used on another stream than the one they were made on, and what a graph
+captured after a warm-up reads once its weight has changed."""
 
 import threading
 
@@ -45,6 +46,88 @@ def test_entry_dropped_inside_an_update(vqx):
     assert q._DECODED_BYTES[7] == 20
     q._release_decoded("a")
     assert q._DECODED_BYTES.pop(7) == 0
+
+
+class HostStream:
+    def synchronize(self):
+        pass
+
+
+@pytest.fixture
+def host_cache(vqx, monkeypatch):
+    """The cache function on CPU tensors: one stream that waits for nothing,
+    captured while the returned dict says so."""
+    q = vqx.ops.quantized
+    state = {"q": q, "capturing": False}
+    monkeypatch.setattr(q._lib, "stream_of", lambda t: 0)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: HostStream())
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: state["capturing"])
+    monkeypatch.setattr(q, "_decoded_fits", lambda nbytes, device: True)
+    return state
+
+
+def cached(state, w):
+    """The cached decode of w, here a copy."""
+    return state["q"]._cached_decode(("test",), (w, None, None), 4, w.clone, True)
+
+
+def test_capture_takes_no_cached_decode(host_cache):
+    w = torch.ones(4)
+    warm = cached(host_cache, w)
+    assert cached(host_cache, w) is warm
+    host_cache["capturing"] = True
+    inside = cached(host_cache, w)
+    assert inside is not warm and cached(host_cache, w) is not inside
+    host_cache["capturing"] = False
+    assert cached(host_cache, w) is warm  # the entry stays for eager calls
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["int8 64 rows", "int8 640 rows", "nf4 40 rows", "outliers"])
+def test_captured_linear_reads_the_weight_as_it_is(vqx, kind):
+    """A graph captured after a warm call, its weight written in place, an
+    eager call on the new weight and the freed memory filled with something
+    else: every replay is the product with the weight of that moment."""
+    print(f"captured linear, {kind}", flush=True)
+    M, N, K, bs = (640 if "640" in kind else 40 if "40" in kind else 64), 384, 512, 64
+    g = torch.Generator(device="cuda").manual_seed(5)
+    nf4 = kind.startswith("nf4")
+    x = torch.randint(-3, 4, (M, K), generator=g, device="cuda").to(torch.bfloat16)
+    sw = torch.ones(N, K // bs, dtype=torch.bfloat16, device="cuda")
+    kw = dict(weight_scale=sw, block_size=bs)
+    if nf4:
+        kw["weight_code"] = torch.arange(-8, 8, device="cuda").to(torch.bfloat16)
+    if kind == "outliers":
+        # one entry of value 5 per row, at column r
+        kw["A_data"] = torch.full((M,), 5.0, dtype=torch.bfloat16, device="cuda")
+        kw["A_indices"] = torch.arange(M, dtype=torch.int32, device="cuda")
+        kw["A_indptr"] = torch.arange(M + 1, dtype=torch.int32, device="cuda")
+
+    def weight():
+        return torch.randint(0 if nf4 else -3, 16 if nf4 else 4, (N, K), generator=g, device="cuda").to(torch.bfloat16)
+
+    def product(w):  # small whole numbers: the product rounds once, the sparse half and its sum once each
+        wd = (kw["weight_code"][w.long()] if nf4 else w).double()
+        y = (x.double() @ wd.t()).to(torch.bfloat16)
+        return y + (5 * wd.t()[:M]).to(torch.bfloat16) if kind == "outliers" else y
+
+    w = weight()
+    for _ in range(2):
+        assert torch.equal(Q.linear_mx(x, w, **kw), product(w))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = Q.linear_mx(x, w, **kw)
+    for step in range(3):
+        w.copy_(weight())
+        graph.replay()
+        assert torch.equal(y, product(w)), f"step {step}, before an eager call"
+        assert torch.equal(Q.linear_mx(x, w, **kw), product(w))
+        fill = [torch.full((N, K), 9.0, dtype=torch.bfloat16, device="cuda") for _ in range(8)]
+        graph.replay()
+        assert torch.equal(y, product(w)), f"step {step}, after an eager call"
+        del fill
 
 
 @pytest.mark.gpu

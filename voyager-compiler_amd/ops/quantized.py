@@ -985,12 +985,26 @@ def _activation_decoded(x, code, scale, block_size):
     return _decode_operand(x, code, scale, block_size)
 
 
+def _capturing(device):
+    """Whether the current stream of ``device`` is being captured."""
+    if device.index is None or device.index == torch.cuda.current_device():
+        return torch.cuda.is_current_stream_capturing()
+    with torch.cuda.device(device):
+        return torch.cuda.is_current_stream_capturing()
+
+
 def _cached_decode(form, deps, nbytes, make, bounded):
     """make() for the weight deps[0] and the code / scale it decodes with,
     cached per weight tensor and form, rebuilt when one of deps changes
     (version counters).  bounded: None instead of a new entry that would take
-    the cache past its share of the device's memory."""
+    the cache past its share of the device's memory.
+
+    A graph being captured gets its own decode, also where the cache holds
+    one: its replays then decode the weight as it stands, and read no memory
+    that a later change of the weight gives back."""
     weight = deps[0]
+    if _capturing(weight.device):
+        return make()
     key = (id(weight), form)
     versions = tuple(None if t is None else (t.data_ptr(), _lib.version_of(t)) for t in deps)
     hit = _DECODED.get(key)
@@ -1004,8 +1018,6 @@ def _cached_decode(form, deps, nbytes, make, bounded):
     if bounded and hit is None and not _decoded_fits(nbytes, weight.device):
         return None
     dense = make()
-    if torch.cuda.is_current_stream_capturing():
-        return dense  # part of the graph being captured (its memory pool): decoded again on each replay
     # a later call may come on another stream: it finds the decode finished
     torch.cuda.current_stream(weight.device).synchronize()
     if hit is None:
