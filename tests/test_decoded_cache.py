@@ -83,6 +83,49 @@ def test_capture_takes_no_cached_decode(host_cache):
     assert cached(host_cache, w) is warm  # the entry stays for eager calls
 
 
+def test_writes_that_are_seen(host_cache):
+    """Through the tensor itself, and another storage put under it.  (A write
+    through .data moves no version counter: such a weight is not rebuilt.)"""
+    w = torch.nn.Parameter(torch.ones(4))
+    first = cached(host_cache, w)
+    with torch.no_grad():
+        w.fill_(2.0)
+    second = cached(host_cache, w)
+    assert second is not first and torch.equal(second, w)
+    w.data = torch.full((4,), 3.0)
+    assert torch.equal(cached(host_cache, w), w)
+
+
+@pytest.mark.parametrize("which", [0, 1, 2])
+def test_inference_tensors_are_not_cached(host_cache, which):
+    """A write in place to a tensor without a version counter is seen, whether
+    it is the weight, its code or its scale."""
+    q = host_cache["q"]
+    deps = [torch.ones(4) for _ in range(3)]
+    with torch.inference_mode():
+        deps[which] = torch.ones(4)
+        for value in (1.0, 2.0):
+            deps[which].fill_(value)
+            got = q._cached_decode(("test",), tuple(deps), 4, lambda: deps[which].clone(), True)
+            assert bool((got == value).all())
+    assert (id(deps[0]), ("test",)) not in q._DECODED
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [64, 640])
+def test_inference_weight_written_in_place(vqx, rows):
+    print(f"inference-mode weight written in place, {rows} rows", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(6)
+    with torch.inference_mode():
+        x = torch.randint(-3, 4, (rows, 512), generator=g, device="cuda").to(torch.bfloat16)
+        w = torch.randint(-3, 4, (384, 512), generator=g, device="cuda").to(torch.bfloat16)
+        sw = torch.ones(384, 16, dtype=torch.bfloat16, device="cuda")
+        for _ in range(3):
+            y = Q.linear_mx(x, w, weight_scale=sw, block_size=32)
+            assert torch.equal(y, (x.double() @ w.double().t()).to(torch.bfloat16))
+            w.add_(1)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["int8 64 rows", "int8 640 rows", "nf4 40 rows", "outliers"])
 def test_captured_linear_reads_the_weight_as_it_is(vqx, kind):

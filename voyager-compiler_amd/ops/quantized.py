@@ -1001,9 +1001,11 @@ def _cached_decode(form, deps, nbytes, make, bounded):
 
     A graph being captured gets its own decode, also where the cache holds
     one: its replays then decode the weight as it stands, and read no memory
-    that a later change of the weight gives back."""
+    that a later change of the weight gives back.  Tensors made under
+    inference mode count no versions, so a write in place would go unseen:
+    they are decoded on every call."""
     weight = deps[0]
-    if _capturing(weight.device):
+    if _capturing(weight.device) or any(t is not None and t.is_inference() for t in deps):
         return make()
     key = (id(weight), form)
     versions = tuple(None if t is None else (t.data_ptr(), _lib.version_of(t)) for t in deps)
