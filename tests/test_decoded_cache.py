@@ -49,19 +49,35 @@ def test_entry_dropped_inside_an_update(vqx):
 
 
 class HostStream:
+    """Counts what the cache asks of a stream."""
+
+    waits, events = 0, 0
+
     def synchronize(self):
-        pass
+        self.waits += 1
+
+    def wait_event(self, event):
+        assert event.recorded is not None and event.recorded is not self
+        self.events += 1
+
+
+class HostEvent:
+    recorded = None
+
+    def record(self, stream):
+        self.recorded = stream
 
 
 @pytest.fixture
 def host_cache(vqx, monkeypatch):
-    """The cache function on CPU tensors: one stream that waits for nothing,
-    captured while the returned dict says so."""
+    """The cache function on CPU tensors, with the current stream and whether
+    it is being captured in the returned dict."""
     q = vqx.ops.quantized
-    state = {"q": q, "capturing": False}
-    monkeypatch.setattr(q._lib, "stream_of", lambda t: 0)
+    state = {"q": q, "capturing": False, "stream": HostStream()}
+    monkeypatch.setattr(q._lib, "stream_of", lambda t: id(state["stream"]))
     monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
-    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: HostStream())
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: state["stream"])
+    monkeypatch.setattr(torch.cuda, "Event", HostEvent)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: state["capturing"])
     monkeypatch.setattr(q, "_decoded_fits", lambda nbytes, device: True)
     return state
@@ -81,6 +97,19 @@ def test_capture_takes_no_cached_decode(host_cache):
     assert inside is not warm and cached(host_cache, w) is not inside
     host_cache["capturing"] = False
     assert cached(host_cache, w) is warm  # the entry stays for eager calls
+
+
+def test_a_new_decode_waits_on_the_device_only(host_cache, monkeypatch):
+    """The host waits for no decode; a call on another stream queues a wait for
+    it there, and the stream is recorded on the decode."""
+    recorded = []
+    monkeypatch.setattr(torch.Tensor, "record_stream", lambda t, stream: recorded.append(stream))
+    w, main = torch.ones(4), host_cache["stream"]
+    first = cached(host_cache, w)
+    assert cached(host_cache, w) is first and (main.waits, main.events) == (0, 0) and not recorded
+    side = host_cache["stream"] = HostStream()
+    assert cached(host_cache, w) is first
+    assert (side.waits, side.events) == (0, 1) and recorded == [side]
 
 
 def test_writes_that_are_seen(host_cache):
@@ -197,3 +226,24 @@ def test_decode_outlives_its_weight_on_another_stream(vqx):
     torch.cuda.synchronize()
     assert torch.equal(y, want)
     del again
+
+
+@pytest.mark.gpu
+def test_side_stream_waits_for_a_decode_under_way(vqx):
+    """The decode is still queued behind other work on the main stream when a
+    product on a side stream takes it from the cache."""
+    print("side stream behind a decode under way", flush=True)
+    M, N, K = 64, 1024, 1024
+    g = torch.Generator(device="cuda").manual_seed(4)
+    x = torch.randint(-3, 4, (M, K), generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randint(-3, 4, (N, K), generator=g, device="cuda").to(torch.bfloat16)
+    sw = torch.ones(N, K // 32, dtype=torch.bfloat16, device="cuda")
+    want = (x.double() @ w.double().t()).to(torch.bfloat16)
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    torch.cuda._sleep(20_000_000)
+    first = Q.linear_mx(x, w, weight_scale=sw, block_size=32)
+    with torch.cuda.stream(side):
+        y = Q.linear_mx(x, w, weight_scale=sw, block_size=32)
+    torch.cuda.synchronize()
+    assert torch.equal(first, want) and torch.equal(y, want)

@@ -1013,19 +1013,23 @@ def _cached_decode(form, deps, nbytes, make, bounded):
     if hit is not None and hit[1] == versions and all(
             (r is None and t is None) or (r is not None and r() is t) for r, t in zip(hit[0], deps)):
         if _lib.stream_of(weight) != hit[3]:
-            # allocated on another stream: its memory is not reused before
-            # the work queued here has read it, even if the weight goes first
-            hit[2].record_stream(torch.cuda.current_stream(weight.device))
+            # made on another stream: the work queued here waits for the
+            # decode, and its memory is not reused before that work has read
+            # it, even if the weight goes first
+            stream = torch.cuda.current_stream(weight.device)
+            stream.wait_event(hit[4])
+            hit[2].record_stream(stream)
         return hit[2]
     if bounded and hit is None and not _decoded_fits(nbytes, weight.device):
         return None
     dense = make()
-    # a later call may come on another stream: it finds the decode finished
-    torch.cuda.current_stream(weight.device).synchronize()
+    # a call on another stream waits for this on the device, not the host here
+    made = torch.cuda.Event()
+    made.record(torch.cuda.current_stream(weight.device))
     if hit is None:
         weakref.finalize(weight, _release_decoded, key)
     _store_decoded(key, (tuple(None if t is None else weakref.ref(t) for t in deps), versions, dense,
-                         _lib.stream_of(weight)))
+                         _lib.stream_of(weight), made))
     return dense
 
 
