@@ -99,6 +99,36 @@ def test_capture_takes_no_cached_decode(host_cache):
     assert cached(host_cache, w) is warm  # the entry stays for eager calls
 
 
+def test_single_use_of_a_wide_weight(host_cache):
+    """Where the product that decodes inside is the faster one for a single
+    use, the second call with the same operands makes the decode, a capture
+    none."""
+    q, w = host_cache["q"], torch.ones(4)
+
+    def call():
+        return q._cached_decode(("test",), (w, None, None), 16, w.clone, True, inside=True)
+
+    assert call() is None
+    host_cache["capturing"] = True
+    assert call() is None
+    host_cache["capturing"] = False
+    kept = call()
+    assert torch.equal(kept, w) and call() is kept
+    w.add_(1)
+    assert call() is None and torch.equal(call(), w)
+    key, before = (id(w), ("test",)), q._DECODED_BYTES[None]
+    del w, call
+    assert key not in q._DECODED and q._DECODED_BYTES[None] == before - 16
+
+
+@pytest.mark.parametrize("M,N,coded,pays", [
+    (128, 12288, False, True), (128, 12289, False, False), (129, 9217, False, False), (256, 9216, False, True),
+    (257, 16384, False, True), (512, 16385, False, False), (513, 1 << 20, False, True), (1, 24576, True, True),
+    (256, 24577, True, False), (257, 1 << 20, True, True)])
+def test_decode_pays_once(vqx, M, N, coded, pays):
+    assert vqx.ops.quantized._decode_pays_once(M, N, coded) == pays
+
+
 def test_a_new_decode_waits_on_the_device_only(host_cache, monkeypatch):
     """The host waits for no decode; a call on another stream queues a wait for
     it there, and the stream is recorded on the decode."""
@@ -156,13 +186,16 @@ def test_inference_weight_written_in_place(vqx, rows):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("kind", ["int8 64 rows", "int8 640 rows", "nf4 40 rows", "outliers"])
+@pytest.mark.parametrize("kind", ["int8 64 rows", "int8 640 rows", "nf4 40 rows", "outliers", "int8 wide",
+                                  "int8 transposed"])
 def test_captured_linear_reads_the_weight_as_it_is(vqx, kind):
     """A graph captured after a warm call, its weight written in place, an
     eager call on the new weight and the freed memory filled with something
     else: every replay is the product with the weight of that moment."""
     print(f"captured linear, {kind}", flush=True)
     M, N, K, bs = (640 if "640" in kind else 40 if "40" in kind else 64), 384, 512, 64
+    if kind == "int8 wide":  # decoded inside the product on the first call and in the graph
+        N = 12416
     g = torch.Generator(device="cuda").manual_seed(5)
     nf4 = kind.startswith("nf4")
     x = torch.randint(-3, 4, (M, K), generator=g, device="cuda").to(torch.bfloat16)
@@ -184,8 +217,8 @@ def test_captured_linear_reads_the_weight_as_it_is(vqx, kind):
         y = (x.double() @ wd.t()).to(torch.bfloat16)
         return y + (5 * wd.t()[:M]).to(torch.bfloat16) if kind == "outliers" else y
 
-    w = weight()
-    for _ in range(2):
+    w = weight().t().contiguous().t() if kind == "int8 transposed" else weight()
+    for _ in range(3):
         assert torch.equal(Q.linear_mx(x, w, **kw), product(w))
     torch.cuda.synchronize()
     graph = torch.cuda.CUDAGraph()

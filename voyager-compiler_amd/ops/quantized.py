@@ -892,7 +892,7 @@ def _store_decoded(key, entry):
     with _DECODED_LOCK:
         old = _DECODED.pop(key, None)
         for e, sign in ((old, -1), (entry, 1)):
-            if e is not None:
+            if e is not None and e[2] is not None:
                 d, n = e[2].device.index, sign * _nbytes(e[2])
                 _DECODED_BYTES[d] = _DECODED_BYTES.get(d, 0) + n
         if entry is not None:
@@ -993,11 +993,13 @@ def _capturing(device):
         return torch.cuda.is_current_stream_capturing()
 
 
-def _cached_decode(form, deps, nbytes, make, bounded):
+def _cached_decode(form, deps, nbytes, make, bounded, inside=False):
     """make() for the weight deps[0] and the code / scale it decodes with,
     cached per weight tensor and form, rebuilt when one of deps changes
     (version counters).  bounded: None instead of a new entry that would take
-    the cache past its share of the device's memory.
+    the cache past its share of the device's memory.  inside: for a single use
+    the product that decodes inside is the faster one, so None where the decode
+    cannot be kept, and on the first call with these deps as they are.
 
     A graph being captured gets its own decode, also where the cache holds
     one: its replays then decode the weight as it stands, and read no memory
@@ -1006,12 +1008,13 @@ def _cached_decode(form, deps, nbytes, make, bounded):
     they are decoded on every call."""
     weight = deps[0]
     if _capturing(weight.device) or any(t is not None and t.is_inference() for t in deps):
-        return make()
+        return None if inside else make()
     key = (id(weight), form)
     versions = tuple(None if t is None else (t.data_ptr(), _lib.version_of(t)) for t in deps)
     hit = _DECODED.get(key)
-    if hit is not None and hit[1] == versions and all(
-            (r is None and t is None) or (r is not None and r() is t) for r, t in zip(hit[0], deps)):
+    seen = hit is not None and hit[1] == versions and all(
+        (r is None and t is None) or (r is not None and r() is t) for r, t in zip(hit[0], deps))
+    if seen and hit[2] is not None:
         if _lib.stream_of(weight) != hit[3]:
             # made on another stream: the work queued here waits for the
             # decode, and its memory is not reused before that work has read
@@ -1020,12 +1023,14 @@ def _cached_decode(form, deps, nbytes, make, bounded):
             stream.wait_event(hit[4])
             hit[2].record_stream(stream)
         return hit[2]
-    if bounded and hit is None and not _decoded_fits(nbytes, weight.device):
+    if bounded and (hit is None or hit[2] is None) and not _decoded_fits(nbytes, weight.device):
         return None
-    dense = make()
-    # a call on another stream waits for this on the device, not the host here
-    made = torch.cuda.Event()
-    made.record(torch.cuda.current_stream(weight.device))
+    dense = made = None
+    if seen or not inside:
+        dense = make()
+        # a call on another stream waits for this on the device, not the host here
+        made = torch.cuda.Event()
+        made.record(torch.cuda.current_stream(weight.device))
     if hit is None:
         weakref.finalize(weight, _release_decoded, key)
     _store_decoded(key, (tuple(None if t is None else weakref.ref(t) for t in deps), versions, dense,
@@ -1033,11 +1038,11 @@ def _cached_decode(form, deps, nbytes, make, bounded):
     return dense
 
 
-def _decoded_weight(weight, code, scale, block_size, kdim, bounded=False):
+def _decoded_weight(weight, code, scale, block_size, kdim):
     """The bf16 decode of a convert-format weight in its own layout, cached
     as the packed NF4 weight is."""
     return _cached_decode(("dense", block_size, kdim), (weight, code, scale), _nbytes(weight),
-                          lambda: _mx_decoded(weight, code, scale, block_size, kdim), bounded)
+                          lambda: _mx_decoded(weight, code, scale, block_size, kdim), False)
 
 
 _DENSE_WS = {}
@@ -1077,12 +1082,27 @@ def _dense_takes(M, N, K):
     return K % 64 == 0 and K > 0 and M > 0 and N > 0 and 2 * M * K < 1 << 32 and 2 * N * K < 1 << 32
 
 
-def _dense_weight_linear(a, a_code, a_scale, w, w_code, w_scale, block_size, bias):
+def _decode_pays_once(M, N, coded):
+    """Whether decoding a weight [N, K] for one product of M rows beats the
+    product that decodes it inside (M <= 512).  That one's time grows with the
+    128 x 128 tiles per CU, the decode's with N K.  Measured, us, decode and
+    dense product / inside, K 4096: M 1, N 4096 32 / 55, 11008 56 / 58, 14336
+    69 / 60, 32000 165 / 77; M 200, N 8192 59 / 60, 11008 67 / 61; M 512, N
+    14336 96 / 111, 28672 229 / 196; with a code table, M 1, N 16384 86 / 120,
+    28672 148 / 128; M 512, N 28672 228 / 271."""
+    tiles = -(-M // 128)
+    if tiles > (2 if coded else _FUSED_DECODE_MAX_TILES):
+        return True
+    return N <= (24576 if coded else (12288, 9216, 16384, 16384)[tiles - 1])
+
+
+def _dense_weight_linear(a, a_code, a_scale, w, w_code, w_scale, block_size, bias, packable):
     """A linear whose weight [N, K] is decoded once (cached) and whose
     activations a [M, K] are decoded by the streaming pass, as one dense
     product; None when the operands fall outside it.  At every M this beats
     decoding the weight in the product's staging (1000 x 4096 x 4096 MXINT8
-    61 -> 45 us, 512 rows 56 -> 28 us of product)."""
+    61 -> 45 us, 512 rows 56 -> 28 us of product).  packable: the other way
+    is the packed weight, not the product that decodes inside."""
     M, K = a.shape
     if w.dim() != 2 or w.shape[1] != K or not _dense_takes(M, w.shape[0], K) or a.device != w.device:
         return None
@@ -1092,7 +1112,12 @@ def _dense_weight_linear(a, a_code, a_scale, w, w_code, w_scale, block_size, bia
                              or bias.device != a.device):
         return None
     if w_code is not None or w_scale is not None:
-        w = _decoded_weight(w, w_code, w_scale, block_size, -1, bounded=True)
+        # rows of K, plainly stored: the product finds a new decode in the caches
+        # (1000 x 4096 x 4096, decode and product 60 -> 53 us)
+        form, src = ("k_last", block_size), w
+        w = _cached_decode(form, (w, w_code, w_scale), _nbytes(w),
+                           lambda: _mx_rows(src, w_code, w_scale, block_size, -1)[0], True,
+                           inside=not packable and not _decode_pays_once(M, w.shape[0], w_code is not None))
         if w is None:
             return None
     if a_code is not None or a_scale is not None:
@@ -1249,7 +1274,7 @@ def linear_mx(input, weight, bias=None, *, input_scale=None, weight_scale=None, 
         if input_scale is None or tuple(input_scale.shape[:-1]) == tuple(input.shape[:-1]):
             s = None if input_scale is None else input_scale.reshape(-1, input_scale.shape[-1])
             dense = _dense_weight_linear(input.reshape(-1, K), input_code, s, weight, weight_code, weight_scale,
-                                         block_size, bias)
+                                         block_size, bias, packable)
             if dense is not None:
                 dense = dense.reshape(*input.shape[:-1], dense.shape[-1])
     if dense is None and packable:
