@@ -85,7 +85,7 @@ def host_cache(vqx, monkeypatch):
 
 def cached(state, w):
     """The cached decode of w, here a copy."""
-    return state["q"]._cached_decode(("test",), (w, None, None), 4, w.clone, True)
+    return state["q"]._cached_decode(("test",), (w, None, None), 4, w.clone)
 
 
 def test_capture_takes_no_cached_decode(host_cache):
@@ -106,7 +106,7 @@ def test_single_use_of_a_wide_weight(host_cache):
     q, w = host_cache["q"], torch.ones(4)
 
     def call():
-        return q._cached_decode(("test",), (w, None, None), 16, w.clone, True, inside=True)
+        return q._cached_decode(("test",), (w, None, None), 16, w.clone, inside=True)
 
     assert call() is None
     host_cache["capturing"] = True
@@ -127,6 +127,14 @@ def test_single_use_of_a_wide_weight(host_cache):
     (256, 24577, True, False), (257, 1 << 20, True, True)])
 def test_decode_pays_once(vqx, M, N, coded, pays):
     assert vqx.ops.quantized._decode_pays_once(M, N, coded) == pays
+
+
+def test_no_entry_where_it_does_not_fit(host_cache, monkeypatch):
+    q, w = host_cache["q"], torch.ones(4)
+    monkeypatch.setattr(q, "_decoded_fits", lambda nbytes, device: False)
+    monkeypatch.setattr(q, "_mx_decoded", lambda t, *rest: t.clone())
+    assert q._decoded_weight(w, None, None, 32, -1) is None
+    assert (id(w), ("dense", 32, -1)) not in q._DECODED
 
 
 def test_a_new_decode_waits_on_the_device_only(host_cache, monkeypatch):
@@ -165,9 +173,31 @@ def test_inference_tensors_are_not_cached(host_cache, which):
         deps[which] = torch.ones(4)
         for value in (1.0, 2.0):
             deps[which].fill_(value)
-            got = q._cached_decode(("test",), tuple(deps), 4, lambda: deps[which].clone(), True)
+            got = q._cached_decode(("test",), tuple(deps), 4, lambda: deps[which].clone())
             assert bool((got == value).all())
     assert (id(deps[0]), ("test",)) not in q._DECODED
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["kc", "ck"])
+@pytest.mark.parametrize("rows", [64, 640])
+def test_no_entry_past_the_share(vqx, monkeypatch, layout, rows):
+    """A weight without a packed form, on either side of the 512 rows up to
+    which the product decodes it inside."""
+    print(f"full cache, {layout}, {rows} rows", flush=True)
+    q = vqx.ops.quantized
+    monkeypatch.setattr(q, "_DECODED_SHARE", 1 << 60)
+    g = torch.Generator(device="cuda").manual_seed(7)
+    x = torch.randint(-3, 4, (rows, 512), generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randint(-3, 4, (384, 512), generator=g, device="cuda").to(torch.bfloat16)
+    sw = torch.ones(384, 16, dtype=torch.bfloat16, device="cuda")
+    want = (x.double() @ w.double().t()).to(torch.bfloat16)
+    if layout == "ck":
+        w, sw = w.t().contiguous(), sw.t().contiguous()
+    before = dict(q._DECODED_BYTES)
+    for _ in range(3):
+        assert torch.equal(Q.linear_mx(x, w, weight_scale=sw, block_size=32, weight_layout=layout), want)
+    assert q._DECODED_BYTES == before
 
 
 @pytest.mark.gpu

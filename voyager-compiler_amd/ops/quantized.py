@@ -870,10 +870,10 @@ def _right_operand(b, code, scale, block_size, stored_kn):
 # probabilities of P V (one column tile).
 _FUSED_DECODE_MAX_TILES = 4
 _DECODED = {}
-# Bytes of cached decodes per device.  A linear that has another way (the
-# packed NF4 product, the decode inside the product) takes it rather than let
-# the cache pass a quarter of the device's memory; a weight's decode is given
-# back with the weight.
+# Bytes of cached decodes per device.  Past a quarter of the device's memory a
+# linear goes another way (the packed NF4 product, the decode inside the
+# product, a decode of its own); a weight's decode is given back with the
+# weight.
 _DECODED_SHARE = 4
 _DECODED_BYTES = {}
 # Reentrant, and the total is updated with no allocation between its read and
@@ -993,12 +993,12 @@ def _capturing(device):
         return torch.cuda.is_current_stream_capturing()
 
 
-def _cached_decode(form, deps, nbytes, make, bounded, inside=False):
+def _cached_decode(form, deps, nbytes, make, inside=False):
     """make() for the weight deps[0] and the code / scale it decodes with,
     cached per weight tensor and form, rebuilt when one of deps changes
-    (version counters).  bounded: None instead of a new entry that would take
-    the cache past its share of the device's memory.  inside: for a single use
-    the product that decodes inside is the faster one, so None where the decode
+    (version counters).  None instead of a new entry that would take the cache
+    past its share of the device's memory.  inside: for a single use the
+    product that decodes inside is the faster one, so None where the decode
     cannot be kept, and on the first call with these deps as they are.
 
     A graph being captured gets its own decode, also where the cache holds
@@ -1023,7 +1023,7 @@ def _cached_decode(form, deps, nbytes, make, bounded, inside=False):
             stream.wait_event(hit[4])
             hit[2].record_stream(stream)
         return hit[2]
-    if bounded and (hit is None or hit[2] is None) and not _decoded_fits(nbytes, weight.device):
+    if (hit is None or hit[2] is None) and not _decoded_fits(nbytes, weight.device):
         return None
     dense = made = None
     if seen or not inside:
@@ -1042,7 +1042,7 @@ def _decoded_weight(weight, code, scale, block_size, kdim):
     """The bf16 decode of a convert-format weight in its own layout, cached
     as the packed NF4 weight is."""
     return _cached_decode(("dense", block_size, kdim), (weight, code, scale), _nbytes(weight),
-                          lambda: _mx_decoded(weight, code, scale, block_size, kdim), False)
+                          lambda: _mx_decoded(weight, code, scale, block_size, kdim))
 
 
 _DENSE_WS = {}
@@ -1116,7 +1116,7 @@ def _dense_weight_linear(a, a_code, a_scale, w, w_code, w_scale, block_size, bia
         # (1000 x 4096 x 4096, decode and product 60 -> 53 us)
         form, src = ("k_last", block_size), w
         w = _cached_decode(form, (w, w_code, w_scale), _nbytes(w),
-                           lambda: _mx_rows(src, w_code, w_scale, block_size, -1)[0], True,
+                           lambda: _mx_rows(src, w_code, w_scale, block_size, -1)[0],
                            inside=not packable and not _decode_pays_once(M, w.shape[0], w_code is not None))
         if w is None:
             return None
@@ -1212,8 +1212,8 @@ def _mx_product(a, a_code, a_scale, b, b_code, b_scale, block_size, b_stored_kn,
         b_code = None
     else:
         if b_coded and not b_inline:
-            b = _decoded_weight(b, b_code, b_scale, block_size, bk) if b_static else \
-                _mx_decoded(b, b_code, b_scale, block_size, bk)
+            kept = _decoded_weight(b, b_code, b_scale, block_size, bk) if b_static else None
+            b = _mx_decoded(b, b_code, b_scale, block_size, bk) if kept is None else kept
             b_code, b_scale = None, None
         bd, bs_, bk_major, bld, _, _ = _right_operand(b, b_code, b_scale, block_size, b_stored_kn)
         if not bk_major and N % 8:
@@ -1653,8 +1653,7 @@ def _spmm(data, indices, indptr, B, B_scale=None, B_code=None, block_size=None, 
     # linear's 142 when done on every call), if it is not taken as it is
     Bt = None
     if b_static and B.ndim == 2 and not (B_code is None and B_scale is None and weight_layout == "ck"):
-        Bt = _cached_decode(("rows", weight_layout, block_size), (B, B_code, B_scale), K * N * out_dtype.itemsize, decode,
-                            bounded=True)
+        Bt = _cached_decode(("rows", weight_layout, block_size), (B, B_code, B_scale), K * N * out_dtype.itemsize, decode)
     if Bt is None:
         Bt = decode()
     out_shape = (*batch_shape, R, N)
