@@ -137,6 +137,21 @@ def test_no_entry_where_it_does_not_fit(host_cache, monkeypatch):
     assert (id(w), ("dense", 32, -1)) not in q._DECODED
 
 
+@pytest.mark.parametrize("capturing", [False, True])
+def test_no_memory_for_a_decode(host_cache, capturing):
+    """The call goes the way that needs none instead of failing."""
+    q, w = host_cache["q"], torch.ones(4)
+    host_cache["capturing"] = capturing
+
+    def make():
+        raise torch.cuda.OutOfMemoryError("out of memory")
+
+    assert q._cached_decode(("test",), (w, None, None), 16, make) is None
+    assert (id(w), ("test",)) not in q._DECODED
+    host_cache["capturing"] = False
+    assert torch.equal(cached(host_cache, w), w)
+
+
 def test_a_new_decode_waits_on_the_device_only(host_cache, monkeypatch):
     """The host waits for no decode; a call on another stream queues a wait for
     it there, and the stream is recorded on the decode."""

@@ -993,11 +993,19 @@ def _capturing(device):
         return torch.cuda.is_current_stream_capturing()
 
 
+def _made(make):
+    try:
+        return make()
+    except torch.cuda.OutOfMemoryError:
+        return None
+
+
 def _cached_decode(form, deps, nbytes, make, inside=False):
     """make() for the weight deps[0] and the code / scale it decodes with,
     cached per weight tensor and form, rebuilt when one of deps changes
     (version counters).  None instead of a new entry that would take the cache
-    past its share of the device's memory.  inside: for a single use the
+    past its share of the device's memory, and where no memory is left for the
+    decode: the caller's other way needs less.  inside: for a single use the
     product that decodes inside is the faster one, so None where the decode
     cannot be kept, and on the first call with these deps as they are.
 
@@ -1008,7 +1016,7 @@ def _cached_decode(form, deps, nbytes, make, inside=False):
     they are decoded on every call."""
     weight = deps[0]
     if _capturing(weight.device) or any(t is not None and t.is_inference() for t in deps):
-        return None if inside else make()
+        return None if inside else _made(make)
     key = (id(weight), form)
     versions = tuple(None if t is None else (t.data_ptr(), _lib.version_of(t)) for t in deps)
     hit = _DECODED.get(key)
@@ -1027,7 +1035,9 @@ def _cached_decode(form, deps, nbytes, make, inside=False):
         return None
     dense = made = None
     if seen or not inside:
-        dense = make()
+        dense = _made(make)
+        if dense is None:
+            return None
         # a call on another stream waits for this on the device, not the host here
         made = torch.cuda.Event()
         made.record(torch.cuda.current_stream(weight.device))
