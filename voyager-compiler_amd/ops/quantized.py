@@ -944,6 +944,16 @@ def _mx_decoded(t, code, scale, block_size, kdim):
     return out.transpose(-2, -1) if flipped else out
 
 
+def _rows_takes(batch, R, C, ld, turned):
+    """Sizes vqx_mx_operand_rows takes for a [batch, R, C] operand as it lies
+    in memory and rows of ld values: items under 4 GiB (32-bit byte offsets),
+    32-bit counts of rows and of 8-value chunks, and, turned, a launch of 256
+    threads per 64 x 64 tile below 2^32 threads."""
+    if 2 * R * C >= 1 << 32 or batch * R >= 1 << 31:
+        return False
+    return batch * -(-ld // 64) * -(-C // 64) < 1 << 24 if turned else batch * R * -(-ld // 8) < 1 << 31
+
+
 def _mx_rows(t, code, scale, block_size, kdim, k_last=True, ld=None):
     """t (bf16, contraction dim kdim = -1 or -2, scales along it) decoded to
     dense bf16 rows of K (k_last) padded with zeros to ld, or rows of the
@@ -1641,8 +1651,9 @@ def _spmm(data, indices, indptr, B, B_scale=None, B_code=None, block_size=None, 
         Bc = B.contiguous()
         if B_code is None and B_scale is None and weight_layout == "ck":
             return Bc
-        if weight_layout == "kc" and out_dtype == torch.bfloat16 and nbB * K * N > 0 and B.ndim >= 2 and (
-                B_code is None or B_code.dtype == torch.bfloat16) and _mx_side_ok(Bc, B_code, B_scale, block_size, -1):
+        if weight_layout == "kc" and out_dtype == torch.bfloat16 and nbB * K * N > 0 and (
+                B_code is None or B_code.dtype == torch.bfloat16) and _mx_side_ok(
+                    Bc, B_code, B_scale, block_size, -1) and _rows_takes(nbB, N, K, N, True):
             return _mx_rows(Bc, B_code, B_scale, block_size, -1, False)
         Bt = torch.empty((nbB, K, N), dtype=out_dtype, device=dev)
         code = None if B_code is None else B_code.reshape(-1).contiguous()
