@@ -37,3 +37,43 @@ def test_spmm_layout(launches, N, K, scaled, route):
     q._spmm(fake(16), fake(16, dtype=torch.int32), fake(rows + 1, dtype=torch.int32), fake(N, K),
             fake(N, K // 64) if scaled else None, None, 64)
     assert names == [route, "vqx_spmm_csr"]
+
+
+# P V of an odd length: P inside the product, V turned; one item of P is 4 GiB
+# from 46341 positions on, and past it the operands decode for the library
+# product, as do more items than a launch holds
+@pytest.mark.parametrize("shape,route", [
+    ((32, 1333, 1333, 128), ["vqx_mx_operand_rows", "vqx_mx_matmul_any"]),
+    ((1, 46337, 46337, 128), ["vqx_mx_operand_rows", "vqx_mx_matmul_any"]),
+    ((1, 50001, 50001, 128), None),
+    ((1, 600, 9000001, 256), None),             # V's item
+    ((1 << 22, 600, 9, 4), None),               # the product's launch
+    ((32, 1333, 128, 1333), ["vqx_mx_operand_rows", "vqx_mx_operand_rows", "vqx_dense_matmul"]),
+    ((1, 16777217, 128, 519), None),            # the left item
+    ((1 << 23, 5, 9, 5), None),                 # the dense product's launch
+    ((1 << 22, 5, 9, 5), ["vqx_mx_operand_rows", "vqx_mx_operand_rows", "vqx_dense_matmul"])])
+def test_batched_products(launches, shape, route):
+    q, names = launches
+    B, M, K, N = shape
+    out = q._mx_product(fake(B, M, K), None, fake(B, M, -(-K // 64)), fake(B, K, N), None, fake(B, -(-K // 64), N), 64,
+                        True, None)
+    assert (None if out is None else names) == route
+    assert route is not None or not names
+
+
+@pytest.mark.filterwarnings("ignore:Accessing the data pointer")
+@pytest.mark.parametrize("B,N,takes", [(32, 1999, True), (1 << 24, 64, False), ((1 << 24) - 1, 64, True),
+                                       (1 << 23, 65, False)])
+def test_few_rows(launches, B, N, takes):
+    q, names = launches
+    out = q._few_rows_product(fake(B, 1, 8), None, None, fake(B, 8, N), None, fake(B, 1, N), 8)
+    assert (out is not None) == takes and names == ["vqx_mx_few_rows"] * takes
+
+
+@pytest.mark.parametrize("turned", [False, True])
+@pytest.mark.parametrize("batch,R,C,ld,takes", [(1, 65536, 32768, 32768, False), (1, 65535, 32768, 32768, True),
+                                                (32768, 65536, 8, 8, None), (1 << 24, 8, 8, 8, None)])
+def test_rows_takes(vqx, batch, R, C, ld, takes, turned):
+    """takes None: the plain pass's row count, the turned one's launch."""
+    got = vqx.ops.quantized._rows_takes(batch, R, C, ld, turned)
+    assert got == (takes if takes is not None else not turned and batch * R < 1 << 31)

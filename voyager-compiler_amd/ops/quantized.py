@@ -954,6 +954,13 @@ def _rows_takes(batch, R, C, ld, turned):
     return batch * -(-ld // 64) * -(-C // 64) < 1 << 24 if turned else batch * R * -(-ld // 8) < 1 << 31
 
 
+def _rows_fit(t, kdim, ld):
+    """Whether _mx_rows takes t into rows of K, ld values each."""
+    flipped = not t.is_contiguous() and t.transpose(-2, -1).is_contiguous()
+    R, C = (t.shape[-1], t.shape[-2]) if flipped else (t.shape[-2], t.shape[-1])
+    return _rows_takes(math.prod(t.shape[:-2]), R, C, ld, (kdim == -1) == flipped)
+
+
 def _mx_rows(t, code, scale, block_size, kdim, k_last=True, ld=None):
     """t (bf16, contraction dim kdim = -1 or -2, scales along it) decoded to
     dense bf16 rows of K (k_last) padded with zeros to ld, or rows of the
@@ -1096,10 +1103,12 @@ def _dense_linear(x2, w, bias):
     return out
 
 
-def _dense_takes(M, N, K):
-    """Shapes vqx_dense_matmul takes: whole 64-deep steps, each operand under
-    4 GiB (its kernel addresses them with 32-bit byte offsets)."""
-    return K % 64 == 0 and K > 0 and M > 0 and N > 0 and 2 * M * K < 1 << 32 and 2 * N * K < 1 << 32
+def _dense_takes(M, N, K, batch=1):
+    """Shapes vqx_dense_matmul takes: whole 64-deep steps, each operand's item
+    under 4 GiB (its kernel addresses them with 32-bit byte offsets), a launch
+    of 256 threads per 128 x 128 tile."""
+    return (K % 64 == 0 and K > 0 and M > 0 and N > 0 and 2 * M * K < 1 << 32 and 2 * N * K < 1 << 32
+            and batch * -(-M // 128) * -(-N // 128) < 1 << 23)
 
 
 def _decode_pays_once(M, N, coded):
@@ -1147,17 +1156,20 @@ def _dense_weight_linear(a, a_code, a_scale, w, w_code, w_scale, block_size, bia
 
 def _dense_rows(t, code, scale, block_size, kdim, K):
     """One operand of vqx_dense_matmul: [batch, rows, ceil(K / 64) * 64]
-    contiguous plain bf16 with K last, t itself where it already is that."""
+    contiguous plain bf16 with K last, t itself where it already is that.
+    None past the decode pass's sizes."""
     if code is None and scale is None and K % 64 == 0:
         r = t if kdim == -1 else t.transpose(-2, -1)
         if r.is_contiguous() and r.data_ptr() % 16 == 0:
             return r.reshape(-1, r.shape[-2], K)
-    return _mx_rows(t, code, scale, block_size, kdim, True, -(-K // 64) * 64)
+    ld = -(-K // 64) * 64
+    return _mx_rows(t, code, scale, block_size, kdim, True, ld) if _rows_fit(t, kdim, ld) else None
 
 
 def _dense_product(a, a_code, a_scale, b, b_code, b_scale, block_size, b_kdim, bias, batch_shape, a_shared, b_shared):
     """The product with both operands decoded ahead (each read by many output
-    tiles), any K, M and N; None past vqx_dense_matmul's 32-bit offsets."""
+    tiles), any K, M and N; None past the sizes vqx_dense_matmul and the
+    decode pass take."""
     M, K = a.shape[-2], a.shape[-1]
     N = b.shape[-2] if b_kdim == -1 else b.shape[-1]
     batch = math.prod(batch_shape)
@@ -1166,10 +1178,12 @@ def _dense_product(a, a_code, a_scale, b, b_code, b_scale, block_size, b_kdim, b
     else:
         rows, nb = M, batch
     Kp = -(-K // 64) * 64
-    if not _dense_takes(rows, N, Kp):
+    if not _dense_takes(rows, N, Kp, nb):
         return None
     ad = _dense_rows(a, a_code, a_scale, block_size, -1, K)
-    bd = _dense_rows(b, b_code, b_scale, block_size, b_kdim, K)
+    bd = None if ad is None else _dense_rows(b, b_code, b_scale, block_size, b_kdim, K)
+    if bd is None:
+        return None
     out = torch.empty(nb, rows, N, dtype=torch.bfloat16, device=a.device)
     ws_bytes = _dense_workspace_bytes(nb, rows, N, Kp, a.device)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=a.device) if ws_bytes else None
@@ -1217,7 +1231,10 @@ def _mx_product(a, a_code, a_scale, b, b_code, b_scale, block_size, b_stored_kn,
     # the product kernel's own rules; a right operand decoded ahead may also
     # be turned to K-major rows of any length
     fits = K >= 8 and N % 4 == 0 and (K % 8 == 0 and (not b_stored_kn or N % 8 == 0))
-    turned = a_inline and b_coded and not b_inline and not fits and K >= 8 and N % 4 == 0
+    ld = -(-K // 8) * 8
+    turned = a_inline and b_coded and not b_inline and not fits and K >= 8 and N % 4 == 0 and \
+        2 * K * M * (batch if b_shared else 1) < 1 << 32 and _rows_fit(b, bk, ld) and \
+        2 * N * ld < 1 << 32 and (1 if b_shared else batch) * row_tiles * -(-N // 128) < 1 << 24
     if not b_static and not turned and not (fits and (a_inline or b_inline)):
         out = _dense_product(a, a_code, a_scale, b, b_code, b_scale, block_size, bk, bias, batch_shape, a_shared, b_shared)
         if out is not None or not fits:
@@ -1227,7 +1244,6 @@ def _mx_product(a, a_code, a_scale, b, b_code, b_scale, block_size, b_stored_kn,
     if (a_code is not None or a_scale is not None) and not a_inline:
         a, a_code, a_scale = _mx_decoded(a, a_code, a_scale, block_size, -1), None, None
     if turned:
-        ld = -(-K // 8) * 8
         bd, bs_, bk_major, bld = _mx_rows(b, b_code, b_scale, block_size, bk, True, ld), None, True, ld
         b_code = None
     else:
@@ -1348,7 +1364,8 @@ def _few_rows_product(a, a_code, a_scale, b, b_code, b_scale, block_size):
     if b.device != dev or not (a.is_contiguous() and b.is_contiguous()):
         return None
     batch = math.prod(sa[:-2])
-    if batch < 1 or 2 * K * N >= 1 << 32:
+    # one item under 4 GiB, a launch of 256 threads per 64 columns below 2^32
+    if batch < 1 or 2 * K * N >= 1 << 32 or batch * -(-N // 64) >= 1 << 24:
         return None
     if a_scale is not None:
         a_scale = a_scale.contiguous()
