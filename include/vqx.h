@@ -475,7 +475,8 @@ int vqx_dense_matmul_workspace_size(int64_t batch, int64_t M, int64_t N, int64_t
  * [rows][K], 0 for [K][rows]) decoded to dense bf16 in the same layout,
  * out contiguous [batch][rows][K] or [batch][K][rows] (16-byte aligned).
  * The host runs it ahead of vqx_mx_matmul for an operand that many output
- * tiles read (decoding once instead of once per tile).  K % 8 == 0;
+ * tiles read (decoding once instead of once per tile).  x aligned and
+ * strided as vqx_mx_matmul takes it; K % 8 == 0;
  * rows % 8 == 0 when k_major = 0.
  */
 int vqx_mx_operand_decode(const VqxMxOperand* x, int64_t batch, int64_t rows, int64_t K, uint16_t* out,

@@ -411,7 +411,7 @@ int vqx_mx_operand_decode(const VqxMxOperand* x, int64_t batch, int64_t rows, in
   if (!x->k_major && rows % 8)
     return set_error(kErrInvalid, "mx_decode: an N-major operand needs a multiple of 8 columns");
   return mx_decode(*reinterpret_cast<const MxOperand*>(x), batch, rows, K, out, x->k_major ? K : rows, false,
-                   true, (hipStream_t)stream);
+                   true, false, (hipStream_t)stream);
 }
 
 int vqx_mx_operand_rows(const VqxMxOperand* x, int64_t batch, int64_t rows, int64_t K, int32_t k_last, uint16_t* out,
@@ -419,7 +419,7 @@ int vqx_mx_operand_rows(const VqxMxOperand* x, int64_t batch, int64_t rows, int6
   g_err[0] = 0;
   if (!x) return set_error(kErrInvalid, "mx_rows: null operand descriptor");
   return mx_decode(*reinterpret_cast<const MxOperand*>(x), batch, rows, K, out, out_ld,
-                   (x->k_major != 0) != (k_last != 0), false, (hipStream_t)stream);
+                   (x->k_major != 0) != (k_last != 0), false, true, (hipStream_t)stream);
 }
 
 int vqx_nf4_pack_weight(const void* weight, int32_t w_dtype, const void* scale, int32_t s_dtype, int64_t N,

@@ -221,7 +221,7 @@ int mx_gemm(const MxOperand& a, const MxOperand& b, const uint16_t* bias, uint16
 int mx_gemv(const MxOperand& a, const MxOperand& b, uint16_t* out, int64_t batch, int64_t M, int64_t N, int64_t K,
             hipStream_t st);
 int mx_decode(const MxOperand& x, int64_t batch, int64_t rows, int64_t K, uint16_t* out, int64_t out_ld, bool turn,
-              bool nt, hipStream_t st);
+              bool nt, bool any, hipStream_t st);  // any: x of any alignment and strides
 
 // vqx_dense_gemm.hip: a [M][K] and b [N][K] plain bf16, strides in elements
 bool dense_gemm_takes(int64_t batch, int64_t M, int64_t N, int64_t K);

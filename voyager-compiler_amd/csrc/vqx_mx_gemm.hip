@@ -962,9 +962,9 @@ int launch_turn(bool srow, const MxOpArgs& o, uint16_t* out, int R, int C, int R
 // x decoded into dense bf16: in its own layout (turn 0, rows padded with zeros
 // to out_ld, a multiple of 8), or with its two dims swapped (turn 1).
 int mx_decode(const MxOperand& x, int64_t batch, int64_t rows, int64_t K, uint16_t* out, int64_t out_ld, bool turn,
-              bool nt, hipStream_t stream) {
+              bool nt, bool any, hipStream_t stream) {
   if (batch < 1 || rows < 1 || K < 1) return set_error(kErrInvalid, "mx_decode: empty operand");
-  int rc = check_operand(x, "mx_decode", false, K, rows, true);
+  int rc = check_operand(x, "mx_decode", false, K, rows, any);
   if (rc) return rc;
   const int64_t R = x.k_major ? rows : K, C = x.k_major ? K : rows, ol = turn ? R : C;
   if (!out || !aligned(out, 16)) return set_error(kErrInvalid, "mx_decode: out must be 16-byte aligned");
