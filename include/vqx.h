@@ -460,7 +460,8 @@ int vqx_mx_few_rows(const uint16_t* a, const uint16_t* a_scale, const uint16_t* 
  * accumulation, bf16 out (contiguous).  a: [M][K] rows lda elements apart,
  * b: [N][K] rows ldb apart; items a_batch_stride / b_batch_stride elements
  * apart (0: shared); both 16-byte aligned, the strides multiples of 8, one
- * item under 4 GiB.  bias: bf16 [N] or NULL.  K % 64 == 0; any M and N.
+ * item under 4 GiB.  bias: bf16 [N] or NULL; out and bias 2-byte aligned.
+ * K % 64 == 0; any M and N.
  * workspace (16-byte aligned): vqx_dense_matmul_workspace_size bytes let a
  * product with few tiles split K; with less (or NULL) it runs whole tiles.
  */

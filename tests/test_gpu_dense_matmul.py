@@ -57,6 +57,28 @@ def test_dense_matmul(vqx, nb, M, N, K, with_bias):
         close(run(vqx, a, b, bias, ws=False)[0], want, mag, K)
 
 
+# an output that starts inside a 16-byte row, in each of the three shapes (K 64
+# short, 200 rows narrow, 2047 rows wide) and with a K split
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(130, 264, 64), (200, 264, 320), (2047, 11008, 320), (100, 264, 4096)])
+@pytest.mark.parametrize("offset", [1, 4])
+def test_dense_matmul_output_alignment(vqx, M, N, K, offset):
+    print(f"dense output offset {offset} M={M} N={N} K={K}", flush=True)
+    L = vqx._lib
+    g = torch.Generator(device="cuda").manual_seed(offset)
+    a = torch.randint(-2, 3, (M, K), generator=g, device="cuda").to(torch.bfloat16)
+    b = torch.randint(-2, 3, (N, K), generator=g, device="cuda").to(torch.bfloat16)
+    flat = torch.full((M * N + offset + 8,), 9.0, dtype=torch.bfloat16, device="cuda")
+    out = flat[offset:offset + M * N]
+    n = ctypes.c_int64(0)
+    L.call("vqx_dense_matmul_workspace_size", 1, M, N, K, ctypes.byref(n))
+    w = torch.empty(max(n.value, 1), dtype=torch.uint8, device="cuda")
+    L.call("vqx_dense_matmul", L.ptr(a), K, 0, L.ptr(b), K, 0, None, L.ptr(out), 1, M, N, K, L.ptr(w), n.value,
+           L.stream_of(a))
+    assert torch.equal(out.view(M, N), (a.float() @ b.float().t()).to(torch.bfloat16))  # whole numbers: one rounding
+    assert bool((flat[:offset] == 9).all()) and bool((flat[offset + M * N:] == 9).all())
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M", [16, 17, 40])
 @pytest.mark.parametrize("fits", [True, False])

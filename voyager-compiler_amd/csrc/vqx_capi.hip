@@ -387,6 +387,7 @@ int vqx_dense_matmul(const uint16_t* a, int64_t lda, int64_t a_batch_stride, con
                      (long long)M, (long long)N, (long long)K);
   if (!aligned(a, 16) || !aligned(b, 16) || lda % 8 || ldb % 8 || a_batch_stride % 8 || b_batch_stride % 8)
     return set_error(kErrInvalid, "dense_matmul: operands must be 16-byte aligned, strides multiples of 8");
+  if (!aligned(out, 2) || !aligned(bias, 2)) return set_error(kErrInvalid, "dense_matmul: out and bias hold bf16 values");
   if (lda < K || ldb < K || a_batch_stride < 0 || b_batch_stride < 0)
     return set_error(kErrInvalid, "dense_matmul: row stride below K or negative batch stride");
   // each item is addressed with 32-bit byte offsets

@@ -327,13 +327,14 @@ __global__ __launch_bounds__(256, S::kOcc) void dense_gemm_kernel(DenseArgs p) {
   constexpr int kChunks = kBN / 8, kRowsOut = 256 / kChunks;  // 16-byte chunks per row; rows per round of the workgroup
   const int c = threadIdx.x % kChunks, nn = pos.n0 + c * 8;
   uint16_t* const ob = p.out + pos.b * (int64_t)p.M * p.N;
+  const bool rows16 = (p.N & 7) == 0 && ((uintptr_t)p.out & 15) == 0;  // every row 16-byte aligned
 #pragma unroll
   for (int q = 0; q < kBM / kRowsOut; ++q) {
     const int r = q * kRowsOut + threadIdx.x / kChunks, m = pos.m0 + r;
     const u32x4 v = *reinterpret_cast<const u32x4*>(lds + r * kOutRow + c * 16);
     if (m < p.M && nn < p.N) {
       uint16_t* const o = ob + (int64_t)m * p.N + nn;
-      if ((p.N & 7) == 0) st_nt(reinterpret_cast<u32x4*>(o), v);
+      if (rows16) st_nt(reinterpret_cast<u32x4*>(o), v);
       else store_any(o, p.N - nn, v);
     }
   }
