@@ -1,9 +1,11 @@
 """GPU: linear_mx / matmul_mx on the operands convert_pt2e writes
 (src/vc/quantization/quantize_pt2e.py:456-508 and the rewrite at :592-645):
 the weight as integer-valued code indices in a bf16 tensor, the 16 NF4 levels
-as weight_code, bf16 scales per 64-element block along K.  These calls run
-the fused dequant MFMA product (the packed operands are built once per weight
-and cached); the result is compared with the oracle's linear_mx / matmul_mx
+as weight_code, bf16 scales per 64-element block along K.  Up to 16 rows, and
+at any number for a weight stored [K, N], these calls run the fused dequant
+MFMA product (the packed operands are built once per weight and cached); other
+linears run the dense product on the weight's decode (made once, cached).  The
+result is compared with the oracle's linear_mx / matmul_mx
 (the reference's decode, then torch CPU bf16 F.linear / matmul) within
 relative tolerance 1e-2, as north_star states for GEMM outputs."""
 
@@ -71,6 +73,17 @@ def fused_only():
         torch.nn.functional.linear, torch.matmul = saved
 
 
+def took(vqx, w):
+    """Which cached form of weight w its calls have made."""
+    q = vqx.ops.quantized
+    forms = {"packed"} if (id(w), False) in q._PACKED else set()
+    return forms | ({"decoded"} if any(k[0] == id(w) for k in q._DECODED) else set())
+
+
+# 16 rows read the packed weight, more its decode
+ROUTES = [(16, "packed"), (64, "decoded")]
+
+
 def test_convert_weight_is_the_nf4_index_table():
     # the convert format's code and index table restate the reference's
     # unique + searchsorted of the nf4 table (quantize_pt2e.py:457-466)
@@ -105,8 +118,8 @@ def test_linear_mx_fused_c5_shape(vqx):
 @pytest.mark.parametrize("M,N,K", [(1, 11008, 4096), (16, 11008, 4096), (5, 200, 512), (300, 384, 1024),
                                    (256, 11008, 4096)])
 def test_linear_mx_fused_matches_oracle(vqx, M, N, K):
-    # M <= 16 runs the skinny kernel (any N), larger M the tile kernel, with
-    # a partial row tile (300) or the stream-K split (256 x 11008)
+    # M <= 16 runs the skinny kernel (any N), larger M the dense product, with
+    # partial row tiles (300)
     print(f"linear_mx fused M={M} N={N} K={K}", flush=True)
     g = torch.Generator().manual_seed(M + N)
     A = torch.randn(M, K, generator=g).to(torch.bfloat16)
@@ -154,10 +167,11 @@ def test_matmul_mx_fused(vqx, layout, shape):
 
 
 @pytest.mark.gpu
-def test_linear_mx_fused_short_code_and_negative_indices(vqx):
+@pytest.mark.parametrize("M,route", ROUTES)
+def test_linear_mx_fused_short_code_and_negative_indices(vqx, M, route):
     # a 9-entry code (fewer than 16 levels), indices as the reference reads
     # them: truncated toward zero, negative ones counting from the end
-    N, K, M = 256, 256, 32
+    N, K = 256, 256
     g = torch.Generator().manual_seed(11)
     code = torch.linspace(-1, 1, 9).to(torch.bfloat16)
     raw = torch.randint(-9, 9, (N, K), generator=g).float()
@@ -165,21 +179,30 @@ def test_linear_mx_fused_short_code_and_negative_indices(vqx):
     idx = raw.to(torch.bfloat16)
     scale = (torch.rand(N, K // 64, generator=g) + 0.5).to(torch.bfloat16)
     A = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    w = idx.cuda()
     with fused_only():
-        out = Q.linear_mx(A.cuda(), idx.cuda(), None, weight_scale=scale.cuda(), weight_code=code.cuda(), block_size=64)
+        out = Q.linear_mx(A.cuda(), w, None, weight_scale=scale.cuda(), weight_code=code.cuda(), block_size=64)
+    assert took(vqx, w) == {route}
     within_tolerance(out, R.linear_mx(A, idx, None, scale, 64, code))
 
 
 @pytest.mark.gpu
-def test_linear_mx_out_of_range_index_takes_unfused_path(vqx):
+@pytest.mark.parametrize("M,route", ROUTES)
+def test_linear_mx_out_of_range_index_takes_unfused_path(vqx, M, route):
     # the reference raises IndexError on an index past the code table; the
-    # packing reports it and the call decodes without the fused kernel, the
-    # bad entry as NaN (only the outputs that read it)
-    N, K, M = 128, 128, 32
+    # packing reports it and the call decodes without the fused kernel (more
+    # than 16 rows decode anyway), the bad entry as NaN (only the outputs that
+    # read it)
+    N, K = 128, 128
     idx, scale, code = random_convert_format(N, K, 12)
     idx[5, 7] = 16.0
     A = torch.randn(M, K, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16)
-    out = Q.linear_mx(A.cuda(), idx.cuda(), None, weight_scale=scale.cuda(), weight_code=code.cuda(), block_size=64)
+    w = idx.cuda()
+    out = Q.linear_mx(A.cuda(), w, None, weight_scale=scale.cuda(), weight_code=code.cuda(), block_size=64)
+    if route == "packed":
+        assert vqx.ops.quantized._PACKED[(id(w), False)].codes is None  # reported
+    else:
+        assert took(vqx, w) == {route}
     o = out.float().cpu()
     assert bool(torch.isnan(o[:, 5]).all())
     keep = torch.ones(N, dtype=torch.bool)
@@ -190,10 +213,11 @@ def test_linear_mx_out_of_range_index_takes_unfused_path(vqx):
 
 
 @pytest.mark.gpu
-def test_linear_mx_fused_repacks_after_weight_update(vqx):
-    # the packed operands are cached per weight and rebuilt when the weight,
-    # its code or its scale change in place (version counters)
-    N, K, M = 256, 512, 64
+@pytest.mark.parametrize("M,route", ROUTES)
+def test_linear_mx_fused_repacks_after_weight_update(vqx, M, route):
+    # the packed operands, and the decode, are cached per weight and rebuilt
+    # when the weight, its code or its scale change in place (version counters)
+    N, K = 256, 512
     idx, scale, code = random_convert_format(N, K, 13)
     A = torch.randn(M, K, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).cuda()
     w, s, c = idx.cuda(), scale.cuda(), code.cuda()
@@ -204,6 +228,7 @@ def test_linear_mx_fused_repacks_after_weight_update(vqx):
     s.mul_(2)
     with fused_only():
         second = Q.linear_mx(A, w, None, weight_scale=s, weight_code=c, block_size=64)
+    assert took(vqx, w) == {route}
     idx2 = idx.clone()
     idx2[:, :64] = 15.0
     within_tolerance(second, R.linear_mx(A.cpu(), idx2, None, scale * 2, 64, code))
@@ -225,12 +250,13 @@ def test_linear_mx_unfusable_operands_still_match(vqx):
 
 
 @pytest.mark.gpu
-def test_linear_mx_fused_offset_views(vqx):
+@pytest.mark.parametrize("M,route", ROUTES)
+def test_linear_mx_fused_offset_views(vqx, M, route):
     # activations cut from a flat buffer at an odd element offset and a bias
     # sliced at an offset that is not a multiple of 4 elements: contiguous
     # views whose storage is not 16- (A) or 8-byte (bias) aligned still run
     # fused and match the oracle
-    N, K, M = 256, 512, 48
+    N, K = 256, 512
     idx, scale, code = random_convert_format(N, K, 15)
     g = torch.Generator().manual_seed(16)
     flat = torch.randn(M * K + 3, generator=g).to(torch.bfloat16).cuda()
@@ -238,17 +264,20 @@ def test_linear_mx_fused_offset_views(vqx):
     bflat = torch.randn(N + 5, generator=g).to(torch.bfloat16).cuda()
     bias = bflat[5:]
     assert x.data_ptr() % 16 and bias.data_ptr() % 8
+    w = idx.cuda()
     with fused_only():
-        out = Q.linear_mx(x, idx.cuda(), bias, weight_scale=scale.cuda(), weight_code=code.cuda(), block_size=64)
+        out = Q.linear_mx(x, w, bias, weight_scale=scale.cuda(), weight_code=code.cuda(), block_size=64)
+    assert took(vqx, w) == {route}
     within_tolerance(out, R.linear_mx(x.cpu(), idx, bias.cpu(), scale, 64, code))
 
 
 @pytest.mark.gpu
-def test_linear_mx_fused_under_inference_mode(vqx):
+@pytest.mark.parametrize("M,forms", [(16, {"packed"}), (64, set())])
+def test_linear_mx_fused_under_inference_mode(vqx, M, forms):
     # operands made under torch.inference_mode carry no version counter; the
     # packed-weight cache keys them on their storage and the call runs fused,
-    # twice (the second from the cache)
-    N, K, M = 256, 512, 32
+    # twice (the second from the cache); more than 16 rows decode on each call
+    N, K = 256, 512
     idx, scale, code = random_convert_format(N, K, 17)
     A = torch.randn(M, K, generator=torch.Generator().manual_seed(18)).to(torch.bfloat16)
     with torch.inference_mode():
@@ -257,5 +286,7 @@ def test_linear_mx_fused_under_inference_mode(vqx):
         with fused_only():
             first = Q.linear_mx(a, w, None, weight_scale=s, weight_code=c, block_size=64)
             second = Q.linear_mx(a, w, None, weight_scale=s, weight_code=c, block_size=64)
+        assert took(vqx, w) == forms
     assert torch.equal(first, second)
+    within_tolerance(first, R.linear_mx(A, idx, None, scale, 64, code))
     within_tolerance(first, R.linear_mx(A, idx, None, scale, 64, code))

@@ -144,8 +144,8 @@ def test_mxint8_linear(vqx, M, N, K):
 @pytest.mark.parametrize("layout", ["kc", "ck"])
 def test_linear_coded_activation_wide_code_weight(vqx, layout):
     """input_code / input_scale on the activation (nf4_6 indices) with a
-    weight of a 40-entry code table and blocks of 32 along K: both decoded in
-    the kernel, batched activations, either weight layout."""
+    weight of a 40-entry code table and blocks of 32 along K, batched
+    activations: the weight decoded once ("kc") or in the kernel ("ck")."""
     print(f"linear coded activation layout={layout}", flush=True)
     N, K, bs = 384, 512, 32
     code_w = torch.linspace(-3, 3, 40).to(torch.bfloat16)
@@ -163,19 +163,23 @@ def test_linear_coded_activation_wide_code_weight(vqx, layout):
 
 
 @pytest.mark.gpu
-def test_linear_coded_activation_nf4_weight_runs_packed_path(vqx):
+@pytest.mark.parametrize("M,packed", [(16, True), (40, False)])
+def test_linear_coded_activation_nf4_weight(vqx, M, packed):
     """A coded activation with a 16-level weight with blocks of 64: the
     activation is decoded by the vqx decode kernel and the product runs the
-    packed-weight kernel; the result still matches."""
-    N, K, M, bs = 256, 512, 40, 64
+    packed-weight kernel, above 16 rows the dense product on the weight's
+    decode."""
+    N, K, bs = 256, 512, 64
     code = nf4_6_code()
     x = int_operand((M, K), 0, 16, 51)
     xs = e5m3_scales((M, blocks(K, bs)), 52)
     w = int_operand((N, K), 0, 16, 53)
     ws = e5m3_scales((N, blocks(K, bs)), 54)
+    wd, q = w.cuda(), vqx.ops.quantized
     with fused_only():
-        got = Q.linear_mx(*cuda(x, w), None, input_scale=xs.cuda(), weight_scale=ws.cuda(), block_size=bs,
+        got = Q.linear_mx(x.cuda(), wd, None, input_scale=xs.cuda(), weight_scale=ws.cuda(), block_size=bs,
                           input_code=code.cuda(), weight_code=code.cuda())
+    assert ((id(wd), False) in q._PACKED) == packed and any(k[0] == id(wd) for k in q._DECODED) != packed
     within_tolerance(got, R.linear_mx(x, w, None, ws, bs, code, xs, code))
 
 

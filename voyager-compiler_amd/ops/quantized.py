@@ -585,9 +585,10 @@ def gwa_fake_quantize(input, axis, block_size, quant_min, quant_max, scale_qmap=
 
 
 # ---------------------------------------------------------------------------
-# linear_mx / matmul_mx  (quantized.py:286-432): a convert-format weight
-# with up to 16 levels and blocks of 64 runs the fused dequant product;
-# other operands decode on the GPU, then the dense product (hipBLASLt).
+# linear_mx / matmul_mx  (quantized.py:286-432): bf16 convert-format operands
+# run this library's products (the packed NF4 weight, the dense product on
+# decoded operands, the products that decode inside); other operands decode on
+# the GPU, then the library GEMM (hipBLASLt).
 # ---------------------------------------------------------------------------
 _CODE_LUTS = {}
 
@@ -1291,11 +1292,13 @@ def _mx_product(a, a_code, a_scale, b, b_code, b_scale, block_size, b_stored_kn,
 def linear_mx(input, weight, bias=None, *, input_scale=None, weight_scale=None, block_size=None,
               input_code=None, weight_code=None, A_data=None, A_indices=None, A_indptr=None,
               weight_layout="kc"):
-    """quantized.py:295-348.  A convert-format weight of up to 16 levels with
-    blocks of 64 along K runs the packed-weight product (the activations
-    decoded first); other bf16 convert-format operands run the product that
-    decodes both inside the kernel; anything else decodes on the GPU and
-    calls the library GEMM."""
+    """quantized.py:295-348.  Up to 16 rows, a convert-format weight of up to
+    16 levels with blocks of 64 along K runs the packed-weight product (the
+    activations decoded first); other bf16 convert-format operands run the
+    dense product on the weight's decode (made once, cached), or, where that
+    cannot be kept or does not fit, the packed product or the one that decodes
+    inside the kernel; anything else decodes on the GPU and calls the library
+    GEMM."""
     assert weight_layout in ("kc", "ck"), weight_layout
     _lib.require_device(input, "linear_mx")
     transposed = weight_layout == "ck"
