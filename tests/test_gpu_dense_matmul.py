@@ -34,8 +34,25 @@ def run(vqx, a, b, bias, ws=True):
     return out, n.value
 
 
-# edges of the 128 x 256 tile and of the 64-deep, three-stage ring (1 to 7
-# steps, with and without a split), row bands, odd columns, several items
+def plan(M, N, K, nb=1):
+    """The tile's columns and the K pieces the product takes on 256 CUs: the
+    estimate of plan_dense (vqx_dense_gemm.hip) restated."""
+    if K <= 128:
+        return "short", 1
+    best = None
+    for shape, cols, step, start in (("wide", 256, 0.82, 3.0), ("narrow", 128, 0.45, 2.5)):
+        tiles, nk = nb * -(-M // 128) * -(-N // cols), K // 64
+        for s in range(1, 17):
+            if s == 1 or 4 * s <= nk:
+                c = -(-tiles * s // 256) * (step * -(-nk // s) + start)
+                c += 4.0 + 0.2 * (128 * cols * 4e-6) * tiles * s if s > 1 else 0.0
+                if best is None or c < best[0]:
+                    best = (c, shape, s)
+    return best[1:]
+
+
+# (1 to 7 steps of the 64-deep, three-stage ring, with and without a split, row
+# bands, odd columns, several items; the narrow and the short shape)
 @pytest.mark.gpu
 @pytest.mark.parametrize("nb,M,N,K", [(1, 1, 8, 64), (1, 128, 256, 128), (1, 129, 257, 192), (1, 127, 255, 256),
                                       (2, 40, 1000, 320), (1, 1100, 264, 384), (3, 130, 33, 448), (1, 17, 7, 1024),
@@ -52,6 +69,29 @@ def test_dense_matmul(vqx, nb, M, N, K, with_bias):
     if with_bias:
         want, mag = want + bias.double(), mag + bias.double().abs()
     got, need = run(vqx, a, b, bias)
+    close(got, want, mag, K)
+    if need:  # the same product without its workspace runs whole tiles
+        close(run(vqx, a, b, bias, ws=False)[0], want, mag, K)
+
+
+# The wide shape: in 5 and 3 pieces of K (its fp32 sums and their reduction),
+# and whole with partial row and column tiles, odd N, and 4, 5 and 7 steps.
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,pieces", [(333, 4096, 11008, 5), (640, 4096, 11008, 3), (333, 4093, 11008, 5),
+                                          (2047, 11003, 320, 1), (1921, 11009, 256, 1), (2047, 11008, 448, 1)])
+def test_dense_matmul_wide(vqx, M, N, K, pieces):
+    print(f"dense wide M={M} N={N} K={K} pieces={pieces}", flush=True)
+    assert torch.cuda.get_device_properties(0).multi_processor_count == 256
+    assert plan(M, N, K) == ("wide", pieces)
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    a = torch.randn(1, M, K, generator=g, device="cuda").to(torch.bfloat16)
+    b = torch.randn(1, N, K, generator=g, device="cuda").to(torch.bfloat16)
+    bias = torch.randn(N, generator=g, device="cuda").to(torch.bfloat16)
+    want = (a[0].double() @ b[0].double().t() + bias.double())[None]
+    mag = (a[0].double().abs() @ b[0].double().abs().t() + bias.double().abs())[None]
+    got, need = run(vqx, a, b, bias)
+    tiles = -(-M // 128) * -(-N // 256)
+    assert need == (tiles * pieces * 128 * 256 * 4 if pieces > 1 else 0)
     close(got, want, mag, K)
     if need:  # the same product without its workspace runs whole tiles
         close(run(vqx, a, b, bias, ws=False)[0], want, mag, K)

@@ -95,3 +95,24 @@ def test_odd_products(vqx, B, M, N, K, coded, form):
     want, mag = torch.matmul(ad, bd.contiguous()), torch.matmul(ad.abs(), bd.abs().contiguous())
     assert got.shape == want.shape
     close(got, want, mag, K)
+
+
+# Every form of the few-row kernel: 64 or 16 columns per workgroup (the first
+# where that gives every CU one), an item's workgroups on one XCD (batches of
+# eight) or in order
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,N,K,cols,one_xcd", [(32, 1999, 128, 64, True), (8, 65, 513, 16, True),
+                                                (35, 520, 77, 64, False), (32, 128, 1999, 16, True),
+                                                (3, 130, 257, 16, False)])
+@pytest.mark.parametrize("M", [1, 2, 4])
+@pytest.mark.parametrize("coded", [False, True])
+def test_few_rows_forms(vqx, B, N, K, cols, one_xcd, M, coded):
+    print(f"few rows B={B} M={M} N={N} K={K} coded={coded}", flush=True)
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    assert (B * -(-N // 64) >= cus) == (cols == 64) and (B % 8 == 0) == one_xcd
+    bs = 32
+    a, code, sa = operand((B, M, K), -1, bs, coded, 3)
+    b, _, sb = operand((B, K, N), -2, bs, coded, 4)
+    got = vqx.ops.quantized._few_rows_product(a, code, sa, b, code, sb, bs)
+    ad, bd = decoded(a, code, sa, bs, -1).double(), decoded(b, code, sb, bs, -2).double()
+    close(got, torch.matmul(ad, bd), torch.matmul(ad.abs(), bd.abs()), K)
