@@ -75,10 +75,9 @@ def host_cache(vqx, monkeypatch):
     q = vqx.ops.quantized
     state = {"q": q, "capturing": False, "stream": HostStream()}
     monkeypatch.setattr(q._lib, "stream_of", lambda t: id(state["stream"]))
-    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: state["stream"])
     monkeypatch.setattr(torch.cuda, "Event", HostEvent)
-    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: state["capturing"])
+    monkeypatch.setattr(torch._C, "_cuda_isCurrentStreamCapturing", lambda: state["capturing"])
     monkeypatch.setattr(q, "_decoded_fits", lambda nbytes, device: True)
     return state
 

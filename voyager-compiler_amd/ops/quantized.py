@@ -1005,10 +1005,10 @@ def _activation_decoded(x, code, scale, block_size):
 
 def _capturing(device):
     """Whether the current stream of ``device`` is being captured."""
-    if device.index is None or device.index == torch.cuda.current_device():
-        return torch.cuda.is_current_stream_capturing()
+    if device.index is None or device.index == torch._C._cuda_getDevice():
+        return torch._C._cuda_isCurrentStreamCapturing()
     with torch.cuda.device(device):
-        return torch.cuda.is_current_stream_capturing()
+        return torch._C._cuda_isCurrentStreamCapturing()
 
 
 def _made(make):
@@ -1032,14 +1032,26 @@ def _cached_decode(form, deps, nbytes, make, inside=False):
     that a later change of the weight gives back.  Tensors made under
     inference mode count no versions, so a write in place would go unseen:
     they are decoded on every call."""
-    weight = deps[0]
-    if _capturing(weight.device) or any(t is not None and t.is_inference() for t in deps):
+    # plain loops: generators in the two calls of an outlier linear, which its
+    # host dispatch bounds, cost it 5 us of 73
+    weight, versions = deps[0], []
+    for t in deps:
+        if t is None:
+            versions.append(None)
+        elif t.is_inference():
+            return None if inside else _made(make)
+        else:
+            versions.append((t.data_ptr(), t._version))
+    if _capturing(weight.device):
         return None if inside else _made(make)
     key = (id(weight), form)
-    versions = tuple(None if t is None else (t.data_ptr(), _lib.version_of(t)) for t in deps)
     hit = _DECODED.get(key)
-    seen = hit is not None and hit[1] == versions and all(
-        (r is None and t is None) or (r is not None and r() is t) for r, t in zip(hit[0], deps))
+    seen = hit is not None and hit[1] == versions
+    if seen:
+        for r, t in zip(hit[0], deps):
+            if r is not None and r() is not t:
+                seen = False
+                break
     if seen and hit[2] is not None:
         if _lib.stream_of(weight) != hit[3]:
             # made on another stream: the work queued here waits for the
@@ -1147,7 +1159,8 @@ def _dense_weight_linear(a, a_code, a_scale, w, w_code, w_scale, block_size, bia
         form, src = ("k_last", block_size), w
         w = _cached_decode(form, (w, w_code, w_scale), _nbytes(w),
                            lambda: _mx_rows(src, w_code, w_scale, block_size, -1)[0],
-                           inside=not packable and not _decode_pays_once(M, w.shape[0], w_code is not None))
+                           inside=not packable and w.shape[0] > 9216 and not _decode_pays_once(
+                               M, w.shape[0], w_code is not None))
         if w is None:
             return None
     if a_code is not None or a_scale is not None:
