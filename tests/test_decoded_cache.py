@@ -101,15 +101,15 @@ def test_capture_takes_no_cached_decode(host_cache):
 def test_single_use_of_a_wide_weight(host_cache):
     """Where the product that decodes inside is the faster one for a single
     use, the second call with the same operands makes the decode, a capture
-    none."""
+    only where that holds for graphs."""
     q, w = host_cache["q"], torch.ones(4)
 
-    def call():
-        return q._cached_decode(("test",), (w, None, None), 16, w.clone, inside=True)
+    def call(inside=True):
+        return q._cached_decode(("test",), (w, None, None), 16, w.clone, inside, True)
 
     assert call() is None
     host_cache["capturing"] = True
-    assert call() is None
+    assert call() is None and torch.equal(call(False), w)
     host_cache["capturing"] = False
     kept = call()
     assert torch.equal(kept, w) and call() is kept

@@ -1018,14 +1018,15 @@ def _made(make):
         return None
 
 
-def _cached_decode(form, deps, nbytes, make, inside=False):
+def _cached_decode(form, deps, nbytes, make, inside=False, inside_eager=False):
     """make() for the weight deps[0] and the code / scale it decodes with,
     cached per weight tensor and form, rebuilt when one of deps changes
     (version counters).  None instead of a new entry that would take the cache
     past its share of the device's memory, and where no memory is left for the
-    decode: the caller's other way needs less.  inside: for a single use the
-    product that decodes inside is the faster one, so None where the decode
-    cannot be kept, and on the first call with these deps as they are.
+    decode: the caller's other way needs less.  inside, inside_eager: for a
+    single use, in a graph and called eagerly, the product that decodes inside
+    is the faster one, so None where the decode cannot be kept, and on the
+    first call with these deps as they are.
 
     A graph being captured gets its own decode, also where the cache holds
     one: its replays then decode the weight as it stands, and read no memory
@@ -1039,7 +1040,7 @@ def _cached_decode(form, deps, nbytes, make, inside=False):
         if t is None:
             versions.append(None)
         elif t.is_inference():
-            return None if inside else _made(make)
+            return None if inside_eager else _made(make)
         else:
             versions.append((t.data_ptr(), t._version))
     if _capturing(weight.device):
@@ -1064,7 +1065,7 @@ def _cached_decode(form, deps, nbytes, make, inside=False):
     if (hit is None or hit[2] is None) and not _decoded_fits(nbytes, weight.device):
         return None
     dense = made = None
-    if seen or not inside:
+    if seen or not inside_eager:
         dense = _made(make)
         if dense is None:
             return None
@@ -1156,11 +1157,14 @@ def _dense_weight_linear(a, a_code, a_scale, w, w_code, w_scale, block_size, bia
     if w_code is not None or w_scale is not None:
         # rows of K, plainly stored: the product finds a new decode in the caches
         # (1000 x 4096 x 4096, decode and product 60 -> 53 us)
-        form, src = ("k_last", block_size), w
+        form, src, N = ("k_last", block_size), w, w.shape[0]
+        inside = not packable and N > 9216 and not _decode_pays_once(M, N, w_code is not None)
+        # below K 1024 the product that decodes inside is no longer than its
+        # dispatch, which the decode would double: first calls 27 us against
+        # 39, the product 15 at K 768 (with a code table 27), 30 (60) at 2048
+        short = not packable and M <= 512 and K < 1024
         w = _cached_decode(form, (w, w_code, w_scale), _nbytes(w),
-                           lambda: _mx_rows(src, w_code, w_scale, block_size, -1)[0],
-                           inside=not packable and w.shape[0] > 9216 and not _decode_pays_once(
-                               M, w.shape[0], w_code is not None))
+                           lambda: _mx_rows(src, w_code, w_scale, block_size, -1)[0], inside, inside or short)
         if w is None:
             return None
     if a_code is not None or a_scale is not None:
