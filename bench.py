@@ -3,11 +3,11 @@
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--only c2] [--no-cpu]
 
 A step is one pass of a hot-path kernel over one batch of synthetic, seeded
-input already resident in HBM.  The headline (``value``) is BASELINE.json
-configs[1]: NF4 block-64 encode of a bf16 4096x11008 weight (C2), in
+input already resident in HBM.  The headline (``value``) is the
+NF4 block-64 encode of a bf16 4096x11008 weight (C2), in
 quantized elements per second over the whole timed region (K back-to-back
-launches between two synchronisations); every other config is reported in
-``configs``.  A bandwidth-bound config cycles its launches through several
+launches between two synchronisations); every other config's time and fraction
+is reported in ``configs``, its full record with ``--details FILE``.  A bandwidth-bound config cycles its launches through several
 copies of its buffers, more than twice the 256 MiB MALL together, so every
 launch streams from HBM (the cold figure, which every fraction uses); the
 warm figure (one buffer set, input left in the MALL by the launch before) is
@@ -47,6 +47,9 @@ def parse():
     ap.add_argument("--no-warm", action="store_true",
                     help="skip the warm-MALL timing pass (one buffer set re-launched), so that a profiler's "
                          "average over every launch of a kernel is the cold figure the bench reports")
+    ap.add_argument("--details", default=None, metavar="FILE",
+                    help="write every config's full record (workload, kernel, bytes, traffic, oracle timing) there; "
+                         "the JSON line holds its times and fractions")
     ap.add_argument("--hbm-ceiling", action="store_true",
                     help="only measure what HBM sustains on this box for each traffic mix, with 1 GiB working sets "
                          "(beyond the 256 MiB MALL): torch's own copy, fill and read kernels, and the C3 e4m3 "
@@ -1182,6 +1185,18 @@ def calibrate_copy():
     print(json.dumps({"calibration": "device copy", "bytes_read": n, "bytes_written": n, "launches": 5}))
 
 
+def short_record(r):
+    """A config's times and fractions to four digits: the whole JSON line has
+    to fit the last few KiB of output that a caller keeps."""
+    keys = ("kernel_ms", "kernel_ms_warm", "step_ms", "hbm_frac", "step_hbm_frac", "mfma_frac")
+    out = {k: float(f"{r[k]:.4g}") for k in keys if r.get(k) is not None}
+    if "mfma_frac" in out:
+        out.pop("hbm_frac", None)
+    if "cpu_oracle" in r:
+        out["cpu_oracle_s"] = float(f"{r['cpu_oracle']['seconds']:.4g}")
+    return out
+
+
 def main():
     a = parse()
     if a.build_probe:
@@ -1298,7 +1313,7 @@ def main():
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "bf16",
-        "data": "synthetic (seeded, BASELINE.json configs)",
+        "data": "synthetic (seeded)",
         "config": {"workload": head["workload"], "block_size": 64, "format": "nf4", "shape": [4096, 11008]},
         "roofline": {"bound": "hbm", "achieved": head["achieved_GBps"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": head["hbm_frac"], "traffic": head["hbm_traffic_bytes"],
@@ -1307,8 +1322,11 @@ def main():
                      "kernel_ms_avg": head["kernel_ms"], "mall": "cold",
                      "buffer_sets": head["buffer_sets"], "kernel_ms_warm": head.get("kernel_ms_warm")},
         "cpu_baseline": cpu,
-        "configs": results,
+        "configs": {k: short_record(r) for k, r in results.items()},
     }
+    if a.details:
+        with open(a.details, "w") as f:
+            json.dump({**out, "configs": results}, f, indent=1)
     print(json.dumps(out))
 
 

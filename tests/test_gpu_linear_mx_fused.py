@@ -7,7 +7,7 @@ MFMA product (the packed operands are built once per weight and cached); other
 linears run the dense product on the weight's decode (made once, cached).  The
 result is compared with the oracle's linear_mx / matmul_mx
 (the reference's decode, then torch CPU bf16 F.linear / matmul) within
-relative tolerance 1e-2, as north_star states for GEMM outputs."""
+relative tolerance 1e-2, the tolerance of GEMM outputs."""
 
 import contextlib
 

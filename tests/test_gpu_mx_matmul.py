@@ -8,8 +8,7 @@ test/test_codegen.py:126-152), MXINT8 linears with blocks of 16
 levels, ragged shapes, broadcast batches, both storage layouts of the right
 operand, and indices outside the code table.  Results are compared with the
 oracle's linear_mx / matmul_mx (the reference's decode, then torch's bf16
-product) within relative tolerance 1e-2, as north_star states for GEMM
-outputs; the library GEMM is made to fail inside the calls, so a pass
+product) within relative tolerance 1e-2, the tolerance of GEMM outputs; the library GEMM is made to fail inside the calls, so a pass
 proves the HIP kernel ran."""
 
 import pytest
