@@ -19,11 +19,13 @@
 // 173 us instead of 158, and the attention scores 101 instead of 70.
 //
 // Three shapes (us; 1000 x 4096 x 4096 / 2048 x 11008 x 4096 / 32 products of
-// 2048 x 2048 x 128):
-//   kWide   BN 256, BK 64, 3 stages of 48 KiB:   38 / 158 / 109
-//   kNarrow BN 128, BK 64, 3 stages of 32 KiB:   30 / 187 / 133
+// 2048 x 2048 x 128; launches on one set of buffers, in parentheses rotating
+// over 600 MB of them, all on one box; boxes differ by 10%, and the pairs of
+// figures elsewhere in this file are each from one box, on one set):
+//   kWide   BN 256, BK 64, 3 stages of 48 KiB:   41 (56) / 147 (171) / 103 (102)
+//   kNarrow BN 128, BK 64, 3 stages of 32 KiB:   31 (41) / 169 (202) / 131 (131)
 //   kShort  BN 256, BK 32, 3 stages of 24 KiB, two workgroups per CU (one
-//           loads while the other stores):       52 / 185 /  70
+//           loads while the other stores):       53 (78) / 182 (212) /  75 (81)
 // What bounds kWide (2048 x 11008 x 4096, 688 tiles = 2.69 rounds of the
 // CUs): per step and CU 1024 cycles of MFMA against 1152 of LDS (96 KiB of
 // fragment reads, 48 KiB of fills, 128 B per cycle) and 768 of the vector
@@ -376,13 +378,14 @@ __global__ __launch_bounds__(256) void dense_reduce_kernel(DenseArgs p) {
 // The shape and K splits of a product: the least of this estimate (us),
 // fitted to measurements on one MI355X.  A full machine takes 0.82 us per
 // step on kWide and 0.45 on kNarrow; a unit's start and output 3 and 2.5; a
-// split 4 for the second launch and 0.2 per MB of fp32 sums.  Measured /
-// estimated: 1000 x 4096 x 4096 kNarrow 30 / 31, kWide in 2 pieces 41 / 40;
-// 512 x 4096 x 4096 kNarrow in 2 pieces 24 / 24, kWide in 4 27 / 27;
-// 333 x 4096 x 11008 kWide in 5 pieces 47 / 42, kNarrow in 2 56 / 48;
-// 2048 x 11008 x 4096 kWide 158 / 167, kNarrow 187 / 189.
+// split 4 for the second launch and 0.2 per MB of fp32 sums.  Measured on one
+// set of buffers / rotating over 600 MB / estimated: 1000 x 4096 x 4096 kNarrow
+// 31 / 41 / 31, kWide in 2 pieces 41 / 46 / 40; 512 x 4096 x 4096 kNarrow in 2
+// pieces 24 / 31 / 24, kWide in 4 27 / 32 / 27; 333 x 4096 x 11008 kWide in 5
+// pieces 38 / 49 / 42, kNarrow in 2 39 / 58 / 48; 2048 x 11008 x 4096 kWide
+// 147 / 171 / 166, kNarrow 169 / 202 / 188.
 // Products of K <= 128 are bound by the output: kShort (the attention scores
-// 70 us against 109 and 133).
+// 75 us against 103 and 131).
 enum ShapeId : int { kShapeWide = 0, kShapeNarrow = 1, kShapeShort = 2 };
 
 struct Plan {
