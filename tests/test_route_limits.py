@@ -6,6 +6,9 @@ import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
 
 
+pytestmark = pytest.mark.filterwarnings("ignore:Accessing the data pointer")
+
+
 @pytest.fixture
 def launches(vqx, monkeypatch):
     """The entry points called, on fake cuda tensors, by name."""
@@ -61,7 +64,6 @@ def test_batched_products(launches, shape, route):
     assert route is not None or not names
 
 
-@pytest.mark.filterwarnings("ignore:Accessing the data pointer")
 @pytest.mark.parametrize("B,N,takes", [(32, 1999, True), (1 << 24, 64, False), ((1 << 24) - 1, 64, True),
                                        (1 << 23, 65, False)])
 def test_few_rows(launches, B, N, takes):
@@ -77,3 +79,21 @@ def test_rows_takes(vqx, batch, R, C, ld, takes, turned):
     """takes None: the plain pass's row count, the turned one's launch."""
     got = vqx.ops.quantized._rows_takes(batch, R, C, ld, turned)
     assert got == (takes if takes is not None else not turned and batch * R < 1 << 31)
+
+
+@pytest.mark.parametrize("batch,M,N,K,coded,eager,graph", [
+    (32, 1, 4096, 128, True, True, True), (32, 4, 1999, 128, True, True, True), (32, 4, 2048, 77, True, True, True),
+    (32, 2, 2048, 128, True, True, False), (32, 3, 2048, 128, True, False, False),
+    (32, 4, 2048, 128, False, True, False), (32, 4, 4096, 128, False, False, False),
+    (32, 4, 128, 2048, False, True, True), (1, 2, 11008, 4096, False, False, False),
+    (1, 4, 11008, 4096, True, True, True), (256, 2, 128, 1024, False, False, False),
+    (96, 2, 128, 1024, False, True, True), (256, 4, 512, 512, False, True, True)])
+def test_few_rows_faster(launches, monkeypatch, batch, M, N, K, coded, eager, graph):
+    q, names = launches
+    for capturing, few in ((False, eager), (True, graph)):
+        monkeypatch.setattr(q, "_capturing", lambda device: capturing)
+        names.clear()
+        code = fake(16) if coded else None
+        q.matmul_mx(fake(batch, M, K), fake(batch, K, N), weight_scale=fake(batch, -(-K // 8), N), weight_code=code,
+                    block_size=8)
+        assert names == (["vqx_mx_few_rows"] if few else ["vqx_mx_matmul"])

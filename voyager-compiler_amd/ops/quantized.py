@@ -1367,9 +1367,25 @@ def linear_mx(input, weight, bias=None, *, input_scale=None, weight_scale=None, 
 _FEW_ROWS, _FEW_ROWS_VALUES = 4, 16384
 
 
+def _few_rows_faster(batch, M, N, K, coded, eager):
+    """Whether 2 to 4 left rows are faster in vqx_mx_few_rows, whose time grows
+    with them, than in the product of 128 x 128 tiles, which takes N and K that
+    are multiples of 8 and, called eagerly, 21 us of dispatch against 12.
+    Kernels, us, few rows of M 2 .. 4 / tiles (with a code table): 32 x 128 x
+    2048 11.8 .. 13.4 / 11.0 (18.7 .. 24.8 / 14.2), 32 x 128 x 4096 20 .. 24 /
+    17 (31 .. 40 / 23), 32 x 2048 x 128 14 .. 16 / 35 (18 .. 22 / 85), 256 x
+    512 x 512 46 .. 50 / 64, 256 x 1024 x 128 29 .. 31 / 23 (36 .. 39 / 48),
+    1 x 4096 x 11008 70 .. 73 / 66 (77 .. 85 / 116)."""
+    if M == 1 or N % 8 or K % 8:
+        return True
+    if K >= 256:
+        return coded or K < 1024 or batch * N < (10240 if K >= 2048 else 16384)
+    return eager and batch * M * K * N <= (20_000_000 if coded else 40_000_000)
+
+
 def _few_rows_product(a, a_code, a_scale, b, b_code, b_scale, block_size):
     """a[*, M, K] . b[*, K, N] with M <= 4 through vqx_mx_few_rows, or None
-    when the operands fall outside it."""
+    when the operands fall outside it or the tiles are faster."""
     sa, sb = a.shape, b.shape
     nd = len(sa)
     if nd < 2 or nd != len(sb):
@@ -1386,6 +1402,8 @@ def _few_rows_product(a, a_code, a_scale, b, b_code, b_scale, block_size):
     batch = math.prod(sa[:-2])
     # one item under 4 GiB, a launch of 256 threads per 64 columns below 2^32
     if batch < 1 or 2 * K * N >= 1 << 32 or batch * -(-N // 64) >= 1 << 24:
+        return None
+    if M > 1 and not _few_rows_faster(batch, M, N, K, b_code is not None, not _capturing(dev)):
         return None
     if a_scale is not None:
         a_scale = a_scale.contiguous()
@@ -1417,7 +1435,8 @@ def matmul_mx(self, other, *, input_scale=None, weight_scale=None, block_size=No
     transposed = weight_layout == "ck"
     dense = None
     a = None
-    if transposed and other.dim() > 2 and _coded(input_code, input_scale, weight_code, weight_scale):
+    if transposed and other.dim() > 2 and self.dim() > 1 and self.shape[-2] <= _FEW_ROWS and \
+            _coded(input_code, input_scale, weight_code, weight_scale):
         dense = _few_rows_product(self, input_code, input_scale, other, weight_code, weight_scale, block_size)
     if dense is None and weight_code is not None and weight_code.numel() <= 16 and other.dim() == 2:
         a = _activation_decoded(self, input_code, input_scale, block_size)
