@@ -97,3 +97,16 @@ def test_few_rows_faster(launches, monkeypatch, batch, M, N, K, coded, eager, gr
         q.matmul_mx(fake(batch, M, K), fake(batch, K, N), weight_scale=fake(batch, -(-K // 8), N), weight_code=code,
                     block_size=8)
         assert names == (["vqx_mx_few_rows"] if few else ["vqx_mx_matmul"])
+
+
+# linears that decode both operands in one launch: a short K, at most 512 rows
+# and outputs, a coded activation
+@pytest.mark.parametrize("M,N,K,coded,inside", [
+    (512, 512, 960, False, True), (513, 512, 960, False, False), (20, 520, 960, False, False),
+    (20, 512, 1024, False, False), (20, 64, 448, True, True), (20, 64, 512, True, False)])
+def test_small_linear(launches, monkeypatch, M, N, K, coded, inside):
+    q, names = launches
+    monkeypatch.setattr(q, "_cached_decode", lambda form, deps, *rest: deps[0])
+    q.linear_mx(fake(M, K), fake(N, K), None, input_scale=fake(M, K // 8), weight_scale=fake(N, K // 8),
+                weight_code=fake(40) if coded else None, block_size=8)
+    assert names == (["vqx_mx_matmul"] if inside else ["vqx_mx_operand_rows", "vqx_dense_matmul"])

@@ -1323,10 +1323,15 @@ def linear_mx(input, weight, bias=None, *, input_scale=None, weight_scale=None, 
     x = None
     packable = weight_code is not None and weight_code.numel() <= 16
     few_rows = packable and input.dim() > 0 and input.numel() <= _PACKED_ROWS * input.shape[-1]
-    if not few_rows and not transposed and _coded(input_code, input_scale, weight_code, weight_scale) \
-            and input.dim() > 0 and input.shape[-1] > 0:
+    K = input.shape[-1] if input.dim() > 0 else 0
+    # a coded activation, a short K and few tiles: the one launch that decodes
+    # both operands is no longer than its dispatch (20 x 64 x 64: 18 us a call
+    # against 24 for the activation's decode and the dense product)
+    one_launch = not packable and K < (1024 if weight_code is None else 512) and weight.shape[0] <= 512 and (
+        input_code is not None or input_scale is not None) and input.numel() <= 512 * K
+    if K > 0 and K % 64 == 0 and not (few_rows or transposed or one_launch) and _coded(
+            input_code, input_scale, weight_code, weight_scale):
         # [M, K] rows against the weight decoded once
-        K = input.shape[-1]
         if input_scale is None or tuple(input_scale.shape[:-1]) == tuple(input.shape[:-1]):
             s = None if input_scale is None else input_scale.reshape(-1, input_scale.shape[-1])
             dense = _dense_weight_linear(input.reshape(-1, K), input_code, s, weight, weight_code, weight_scale,
@@ -1341,7 +1346,6 @@ def linear_mx(input, weight, bias=None, *, input_scale=None, weight_scale=None, 
             and weight.dim() == 2 and input.shape[-1] > 0 and (
                 input_scale is None or tuple(input_scale.shape[:-1]) == tuple(input.shape[:-1])):
         # the activation's rows as one [M, K] product
-        K = input.shape[-1]
         a = input.reshape(-1, K)
         s = None if input_scale is None else input_scale.reshape(a.shape[0], input_scale.shape[-1])
         dense = _mx_product(a, input_code, s, weight, weight_code, weight_scale, block_size, transposed, bias,
