@@ -61,3 +61,40 @@ def test_table_kernel(vqx, rows, cols, bs, mode):
     ws, wq = R.quantize_mx(x, table, [-1], bs, qmax, mode == "pow2", smap)
     assert_bitexact(s, ws, "scales")
     assert_bitexact(q, wq, "values")
+
+
+# Every set of outputs the C entry point can ask of the kernel, against the same
+# rows in calls below the size from which the table is kept in LDS
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode", ["absmax", "absmax/64", "pow2"])
+@pytest.mark.parametrize("outputs", ["fq", "values fq"])
+def test_table_kernel_fake_quant(vqx, mode, outputs):
+    print(f"table kernel {outputs} {mode}", flush=True)
+    L, q = vqx._lib, vqx.ops.quantized
+    rows, cols, bs = 1311, 1664, 32
+    x = every_pattern(rows * cols, 9).reshape(rows, cols).cuda()
+    d, keep = q._table_desc(random_table(3).cuda(), x.device)
+    qmax, shift = (64.0 if "/" in mode else 31.0), 8
+
+    def call(x):
+        n = x.numel()
+        out = {k: torch.zeros(n, dtype=torch.bfloat16, device="cuda") for k in outputs.split()}
+        scale = torch.zeros(n // bs, dtype=torch.bfloat16, device="cuda")
+        scale32 = torch.zeros(n // bs, dtype=torch.float32, device="cuda")
+        e8m0 = torch.zeros(n // bs, dtype=torch.uint8, device="cuda") if mode == "pow2" else None
+        L.call("vqx_mx_quantize", L.ptr(x), L.BF16, x.shape[0], cols, 1, bs, L.ctypes.byref(d), 0 if mode == "pow2" else 1,
+               shift, qmax, None, L.ptr(scale), L.ptr(scale32), L.ptr(e8m0), L.ptr(out.get("values")),
+               L.ptr(out.get("fq")), None, 0, L.stream_of(x))
+        return [out[k].view(torch.int16) for k in out] + [scale.view(torch.int16), scale32.view(torch.int32)] + (
+            [] if e8m0 is None else [e8m0])
+
+    got = call(x)
+    parts = [call(x[i:i + 400].contiguous()) for i in range(0, rows, 400)]
+    for g, w in zip(got, [torch.cat(p) for p in zip(*parts)]):
+        if g.dtype == torch.int16:  # any NaN is as good as another
+            f, h = g.view(torch.bfloat16), w.view(torch.bfloat16)
+            same = (g == w) | (f.isnan() & h.isnan())
+        else:
+            same = (g == w) | ((g & 0x7FFFFFFF) > 0x7F800000) & ((w & 0x7FFFFFFF) > 0x7F800000) \
+                if g.dtype == torch.int32 else g == w
+        assert bool(same.all()), int((~same).sum())
