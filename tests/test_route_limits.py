@@ -99,6 +99,17 @@ def test_few_rows_faster(launches, monkeypatch, batch, M, N, K, coded, eager, gr
         assert names == (["vqx_mx_few_rows"] if few else ["vqx_mx_matmul"])
 
 
+# a plain right operand: read in place by up to 512 rows of an item, else turned
+@pytest.mark.parametrize("M,N,route", [
+    (100, 4096, ["vqx_mx_operand_decode", "vqx_mx_matmul"]), (512, 2048, ["vqx_mx_operand_decode", "vqx_mx_matmul"]),
+    (513, 2048, ["vqx_mx_operand_rows", "vqx_mx_operand_rows", "vqx_dense_matmul"]),
+    (100, 4095, ["vqx_mx_operand_rows", "vqx_mx_operand_rows", "vqx_dense_matmul"])])
+def test_plain_right_operand(launches, M, N, route):
+    q, names = launches
+    q.matmul_mx(fake(4, M, 512), fake(4, 512, N), input_scale=fake(4, M, 8), block_size=64)
+    assert names == route
+
+
 # linears that decode both operands in one launch: a short K, at most 512 rows
 # and outputs, a coded activation
 @pytest.mark.parametrize("M,N,K,coded,inside", [

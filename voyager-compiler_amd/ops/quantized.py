@@ -1250,10 +1250,13 @@ def _mx_product(a, a_code, a_scale, b, b_code, b_scale, block_size, b_stored_kn,
     # be turned to K-major rows of any length
     fits = K >= 8 and N % 4 == 0 and (K % 8 == 0 and (not b_stored_kn or N % 8 == 0))
     ld = -(-K // 8) * 8
+    # a plain right operand that few tiles read is read in place too (4 items of
+    # 100 x 512 x 4096 14 us, turned for the dense product 25)
+    in_place = fits and (a_inline or b_inline or (not b_coded and row_tiles <= _FUSED_DECODE_MAX_TILES))
     turned = a_inline and b_coded and not b_inline and not fits and K >= 8 and N % 4 == 0 and \
         2 * K * M * (batch if b_shared else 1) < 1 << 32 and _rows_fit(b, bk, ld) and \
         2 * N * ld < 1 << 32 and (1 if b_shared else batch) * row_tiles * -(-N // 128) < 1 << 24
-    if not b_static and not turned and not (fits and (a_inline or b_inline)):
+    if not b_static and not turned and not in_place:
         out = _dense_product(a, a_code, a_scale, b, b_code, b_scale, block_size, bk, bias, batch_shape, a_shared, b_shared)
         if out is not None or not fits:
             return out
