@@ -38,7 +38,7 @@ def plan(M, N, K, nb=1):
     """The tile's columns and the K pieces the product takes on 256 CUs: the
     estimate of plan_dense (vqx_dense_gemm.hip) restated."""
     if K <= 128:
-        return "short", 1
+        return ("narrow" if nb * -(-M // 128) * -(-N // 128) <= 256 else "short"), 1
     best = None
     for shape, cols, step, start in (("wide", 256, 0.82, 3.0), ("narrow", 128, 0.45, 2.5)):
         tiles, nk = nb * -(-M // 128) * -(-N // cols), K // 64
@@ -56,10 +56,12 @@ def plan(M, N, K, nb=1):
 @pytest.mark.gpu
 @pytest.mark.parametrize("nb,M,N,K", [(1, 1, 8, 64), (1, 128, 256, 128), (1, 129, 257, 192), (1, 127, 255, 256),
                                       (2, 40, 1000, 320), (1, 1100, 264, 384), (3, 130, 33, 448), (1, 17, 7, 1024),
-                                      (1, 333, 512, 4096), (1, 64, 2, 11008), (1, 2300, 4104, 64)])
+                                      (1, 333, 512, 4096), (1, 64, 2, 11008), (1, 2300, 4104, 64),
+                                      (1, 2048, 2048, 128), (1, 2049, 2048, 128), (5, 1100, 1001, 64),
+                                      (5, 1001, 1100, 128)])
 @pytest.mark.parametrize("with_bias", [False, True])
 def test_dense_matmul(vqx, nb, M, N, K, with_bias):
-    print(f"dense nb={nb} M={M} N={N} K={K} bias={with_bias}", flush=True)
+    print(f"dense nb={nb} M={M} N={N} K={K} bias={with_bias} plan={plan(M, N, K, nb)}", flush=True)
     g = torch.Generator(device="cuda").manual_seed(M * 7 + N)
     a = torch.randn(nb, M, K, generator=g, device="cuda").to(torch.bfloat16)
     b = torch.randn(nb, N, K, generator=g, device="cuda").to(torch.bfloat16)
@@ -100,7 +102,7 @@ def test_dense_matmul_wide(vqx, M, N, K, pieces):
 # an output that starts inside a 16-byte row, in each of the three shapes (K 64
 # short, 200 rows narrow, 2047 rows wide) and with a K split
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(130, 264, 64), (200, 264, 320), (2047, 11008, 320), (100, 264, 4096)])
+@pytest.mark.parametrize("M,N,K", [(2300, 4104, 64), (200, 264, 320), (2047, 11008, 320), (100, 264, 4096)])
 @pytest.mark.parametrize("offset", [1, 4])
 def test_dense_matmul_output_alignment(vqx, M, N, K, offset):
     print(f"dense output offset {offset} M={M} N={N} K={K}", flush=True)

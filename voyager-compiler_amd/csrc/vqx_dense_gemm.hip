@@ -385,7 +385,9 @@ __global__ __launch_bounds__(256) void dense_reduce_kernel(DenseArgs p) {
 // pieces 38 / 49 / 42, kNarrow in 2 39 / 58 / 48; 2048 x 11008 x 4096 kWide
 // 147 / 171 / 166, kNarrow 169 / 202 / 188.
 // Products of K <= 128 are bound by the output: kShort (the attention scores
-// 75 us against 103 and 131).
+// 75 us against 103 and 131), or kNarrow while its tiles are one round of the
+// CUs (one 2048 x 2048 x 128 6.5 us against 7.8, 12 x 197 x 197 x 64 5.4
+// against 7.6; at 180 kShort tiles, 12 x 577 x 577 x 64, 11.2 against 11.0).
 enum ShapeId : int { kShapeWide = 0, kShapeNarrow = 1, kShapeShort = 2 };
 
 struct Plan {
@@ -399,8 +401,12 @@ int64_t tiles_of(int64_t batch, int64_t M, int64_t N) {
 }
 
 Plan plan_dense(int64_t batch, int64_t M, int64_t N, int64_t K, bool may_split) {
-  if (K <= 128) return {kShapeShort, 1, tiles_of<kShort>(batch, M, N)};
   const int64_t nk = K / 64, cus = num_cus();
+  if (K <= 128) {
+    const int64_t narrow = tiles_of<kNarrow>(batch, M, N);
+    if (narrow <= cus) return {kShapeNarrow, 1, narrow};
+    return {kShapeShort, 1, tiles_of<kShort>(batch, M, N)};
+  }
   Plan best{kShapeWide, 1, 0};
   double cost = 0.0;
   for (int shape = kShapeWide; shape <= kShapeNarrow; ++shape) {
