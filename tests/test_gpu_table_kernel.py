@@ -40,7 +40,8 @@ def random_table(seed):
 # either side of the size from which the table is kept in LDS, a tail of
 # groups past the last whole 1024 elements, every block size, both scales
 @pytest.mark.gpu
-@pytest.mark.parametrize("rows,cols", [(2049, 1024), (1023, 2048), (1311, 1664)])
+@pytest.mark.parametrize("rows,cols", [(2049, 1024), (1023, 2048), (1311, 1664), (2303, 1024), (2305, 1024),
+                                       (1431, 1664)])
 @pytest.mark.parametrize("bs,mode", [(16, "absmax"), (32, "pow2"), (64, "qmap"), (128, "absmax"), (16, "qmap"),
                                      (64, "pow2"), (128, "pow2"), (16, "absmax/1"), (32, "absmax/64"),
                                      (128, "absmax/1")])
@@ -71,7 +72,7 @@ def test_table_kernel(vqx, rows, cols, bs, mode):
 def test_table_kernel_fake_quant(vqx, mode, outputs):
     print(f"table kernel {outputs} {mode}", flush=True)
     L, q = vqx._lib, vqx.ops.quantized
-    rows, cols, bs = 1311, 1664, 32
+    rows, cols, bs = 1431, 1664, 32
     x = every_pattern(rows * cols, 9).reshape(rows, cols).cuda()
     d, keep = q._table_desc(random_table(3).cuda(), x.device)
     qmax, shift = (64.0 if "/" in mode else 31.0), 8

@@ -1095,8 +1095,9 @@ __global__ __launch_bounds__(kMxLutThreads) void mx_lut_kernel(const uint16_t* _
 // an element is its quotient's bf16 rounding and one 2-byte LDS read.  Reading
 // the table from the L2 instead bounds mx_group_kernel (2048 x 11008, nf4_6
 // index table: 34 us against 20, 4.5 TB/s); filling LDS costs about 3 us, so
-// inputs below kTableMin elements keep the gather (2^20 elements 4.6 us
-// against 4.9, 2^21 5.7 both, 2^22 8.6 against 6.3, 2^24 26.9 against 15.7).
+// inputs below kTableMin elements keep the gather (us a launch in a graph,
+// gather / LDS: 2^21 elements 6.5-6.7 / 6.8-7.0, 9 * 2^18 7.3-7.9 / 6.8-7.0,
+// 2^22 8.9-9.7 / 7.2-7.4, 2^23 14.8-15.9 / 9.9-10.3, 2^26 100-108 / 53-55).
 //
 // Quotients: power-of-two scales divide by an exact multiplication.  Absmax
 // scales multiply by v_rcp_f32, which rounds to the bf16 of the reference's
@@ -1105,7 +1106,7 @@ __global__ __launch_bounds__(kMxLutThreads) void mx_lut_kernel(const uint16_t* _
 // on one, and its conversion is left to f2bf): a group whose smallest nonzero
 // magnitude divides to less than 2^-120, or whose scale or maximum is extreme,
 // NaN or Inf, divides exactly.
-constexpr int kTableMin = 1 << 21;
+constexpr int kTableMin = 9 << 18;
 
 template <int LPB, bool ABSMAX, int WANT>
 __global__ __launch_bounds__(kMxLutThreads) void mx_table_kernel(const uint16_t* __restrict__ x, int64_t ngroups,
