@@ -106,8 +106,25 @@ def test_few_rows_faster(launches, monkeypatch, batch, M, N, K, coded, eager, gr
     (100, 4095, ["vqx_mx_operand_rows", "vqx_mx_operand_rows", "vqx_dense_matmul"])])
 def test_plain_right_operand(launches, M, N, route):
     q, names = launches
-    q.matmul_mx(fake(4, M, 512), fake(4, 512, N), input_scale=fake(4, M, 8), block_size=64)
+    q.matmul_mx(fake(4, M, 1024), fake(4, 1024, N), input_scale=fake(4, M, 16), block_size=64)
     assert names == route
+
+
+# decode passes ahead of the dense product or of the tiles, either side of each
+# line: short K by tiles, long K, a plain left and a plain right operand
+@pytest.mark.parametrize("B,M,K,N,coded,dense", [
+    (12, 768, 64, 768, "ab", False), (16, 2048, 64, 2048, "ab", True), (12, 640, 128, 640, "ab", False),
+    (12, 1024, 128, 1024, "ab", True), (1, 520, 256, 520, "ab", True), (1, 520, 248, 520, "ab", False),
+    (31, 1024, 128, 1024, "b", False), (32, 1024, 128, 1024, "b", True), (64, 2048, 64, 2048, "b", False),
+    (1, 520, 256, 520, "b", True), (32, 2048, 2048, 128, "b", False), (12, 1024, 1024, 64, "b", True),
+    (32, 1024, 128, 1024, "a", False), (16, 2048, 128, 2048, "a", True), (1, 1024, 1024, 1024, "a", True),
+    (8, 1024, 512, 1024, "a", False), (1, 1024, 512, 1024, "a", True), (12, 768, 64, 767, "ab", True)])
+def test_dense_or_tiles(launches, B, M, K, N, coded, dense):
+    q, names = launches
+    sa = fake(B, M, -(-K // 8)) if "a" in coded else None
+    sb = fake(B, -(-K // 8), N) if "b" in coded else None
+    q.matmul_mx(fake(B, M, K), fake(B, K, N), input_scale=sa, weight_scale=sb, block_size=8)
+    assert names[-1] == ("vqx_dense_matmul" if dense else "vqx_mx_matmul")
 
 
 # linears that decode both operands in one launch: a short K, at most 512 rows

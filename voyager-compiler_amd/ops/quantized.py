@@ -1211,6 +1211,24 @@ def _dense_product(a, a_code, a_scale, b, b_code, b_scale, block_size, b_kdim, b
     return out.reshape(*batch_shape, M, N)
 
 
+def _dense_faster(tiles, N, K, a_coded, b_coded, b_k_major):
+    """Whether decode passes and the dense product beat decode passes and the
+    tile product (128 x 128 tiles, ``tiles`` of them in all) where both take the
+    shape.  Kernels in a graph, us, dense / tiles; both coded: 12 x 768 x 64 x
+    768 14.6 / 11.8, 12 x 2048 x 64 x 2048 42.9 / 42.3, 32 of it 74 / 91, 12 x
+    640 x 128 x 640 17.7 / 17.2, 12 x 1024 x 128 x 1024 21.0 / 21.7, 32 of it
+    39 / 48, 32 x 640 x 256 x 640 34 / 39.  A plain left operand: 12 x 1024 x
+    128 x 1024 16.7 / 16.6, 32 of it 33 / 38, 32 x 2048 x 2048 x 128 91 / 82,
+    12 x 1024 x 1024 x 64 16.6 / 19.2.  A plain right one, which only the dense
+    product needs turned: 32 x 1024 x 128 x 1024 38.5 / 38.3, 2048 of it 96 /
+    113, 8 x 1024 x 512 x 1024 30 / 24, 1 x 1024 x 1024 x 1024 18.5 / 19.6."""
+    if not a_coded:
+        return (K >= 768 and tiles <= 128) if N <= 512 else (K >= 256 or (K > 64 and tiles >= 2048))
+    if b_coded or b_k_major:
+        return K >= 256 or tiles >= (768 if K > 64 else 4096)
+    return K >= 1024 or (K >= 512 and tiles < 128) or (K > 64 and tiles >= 4096)
+
+
 def _mx_product(a, a_code, a_scale, b, b_code, b_scale, block_size, b_stored_kn, bias, b_static=False):
     """A'[*, M, K] . B' on bf16 operands with scales along K, or None when the
     operands fall outside it.  b: [*, K, N] when b_stored_kn, else [*, N, K];
@@ -1218,9 +1236,9 @@ def _mx_product(a, a_code, a_scale, b, b_code, b_scale, block_size, b_stored_kn,
     decode is cached when it is decoded ahead of the product).
 
     An operand that at most _FUSED_DECODE_MAX_TILES output tiles read is
-    decoded inside the product (vqx_mx_matmul); when neither is, or the
-    product's alignment rules refuse the shape, both are decoded ahead and the
-    dense product runs."""
+    decoded inside the product (vqx_mx_matmul); when neither is, both are
+    decoded ahead for it or, where that is faster or its alignment rules refuse
+    the shape, for the dense product."""
     bk = -2 if b_stored_kn else -1
     if not (_mx_side_ok(a, a_code, a_scale, block_size, -1) and _mx_side_ok(b, b_code, b_scale, block_size, bk)):
         return None
@@ -1242,7 +1260,8 @@ def _mx_product(a, a_code, a_scale, b, b_code, b_scale, block_size, b_stored_kn,
     batch = math.prod(batch_shape)
     if batch < 1:
         return None
-    a_inline = (a_code is not None or a_scale is not None) and -(-N // 128) <= _FUSED_DECODE_MAX_TILES
+    a_coded = a_code is not None or a_scale is not None
+    a_inline = a_coded and -(-N // 128) <= _FUSED_DECODE_MAX_TILES
     row_tiles = -(-(M * (batch if b_shared else 1)) // 128)
     b_coded = b_code is not None or b_scale is not None
     b_inline = b_coded and row_tiles <= _FUSED_DECODE_MAX_TILES
@@ -1256,13 +1275,15 @@ def _mx_product(a, a_code, a_scale, b, b_code, b_scale, block_size, b_stored_kn,
     turned = a_inline and b_coded and not b_inline and not fits and K >= 8 and N % 4 == 0 and \
         2 * K * M * (batch if b_shared else 1) < 1 << 32 and _rows_fit(b, bk, ld) and \
         2 * N * ld < 1 << 32 and (1 if b_shared else batch) * row_tiles * -(-N // 128) < 1 << 24
-    if not b_static and not turned and not in_place:
+    if not b_static and not turned and not in_place and not (fits and not _dense_faster(
+            row_tiles * -(-N // 128) * (1 if b_shared else batch), N, K, a_coded, b_coded,
+            (b.transpose(-2, -1) if b_stored_kn else b).is_contiguous())):
         out = _dense_product(a, a_code, a_scale, b, b_code, b_scale, block_size, bk, bias, batch_shape, a_shared, b_shared)
         if out is not None or not fits:
             return out
     if not fits and not turned:
         return None
-    if (a_code is not None or a_scale is not None) and not a_inline:
+    if a_coded and not a_inline:
         a, a_code, a_scale = _mx_decoded(a, a_code, a_scale, block_size, -1), None, None
     if turned:
         bd, bs_, bk_major, bld = _mx_rows(b, b_code, b_scale, block_size, bk, True, ld), None, True, ld
