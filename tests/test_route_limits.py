@@ -127,11 +127,12 @@ def test_dense_or_tiles(launches, B, M, K, N, coded, dense):
     assert names[-1] == ("vqx_dense_matmul" if dense else "vqx_mx_matmul")
 
 
-# linears that decode both operands in one launch: a short K, at most 512 rows
-# and outputs, a coded activation
+# linears that decode both operands in one launch (the weight ahead above 512
+# rows): a short K, at most 512 outputs and one round of tiles, a coded activation
 @pytest.mark.parametrize("M,N,K,coded,inside", [
-    (512, 512, 960, False, True), (513, 512, 960, False, False), (20, 520, 960, False, False),
-    (20, 512, 1024, False, False), (20, 64, 448, True, True), (20, 64, 512, True, False)])
+    (512, 512, 1024, False, True), (512, 512, 1088, False, False), (513, 512, 960, False, True),
+    (8192, 512, 960, False, True), (8193, 512, 960, False, False), (20, 520, 960, False, False),
+    (20, 64, 512, True, True), (20, 64, 576, True, False), (513, 64, 576, True, True)])
 def test_small_linear(launches, monkeypatch, M, N, K, coded, inside):
     q, names = launches
     monkeypatch.setattr(q, "_cached_decode", lambda form, deps, *rest: deps[0])

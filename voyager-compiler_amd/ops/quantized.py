@@ -1348,11 +1348,14 @@ def linear_mx(input, weight, bias=None, *, input_scale=None, weight_scale=None, 
     packable = weight_code is not None and weight_code.numel() <= 16
     few_rows = packable and input.dim() > 0 and input.numel() <= _PACKED_ROWS * input.shape[-1]
     K = input.shape[-1] if input.dim() > 0 else 0
-    # a coded activation, a short K and few tiles: the one launch that decodes
-    # both operands is no longer than its dispatch (20 x 64 x 64: 18 us a call
-    # against 24 for the activation's decode and the dense product)
-    one_launch = not packable and K < (1024 if weight_code is None else 512) and weight.shape[0] <= 512 and (
-        input_code is not None or input_scale is not None) and input.numel() <= 512 * K
+    # a coded activation, a short K and tiles for one round of the CUs: the one
+    # launch that decodes both operands (the weight too up to 512 rows) is no
+    # longer than its dispatch (20 x 64 x 64 18 us a call against 24 for the
+    # activation's decode and the dense product, 100 x 1024 x 512 23 against 29)
+    one_launch = not packable and 0 < K <= 1024 and weight.shape[0] <= 512 and (
+        input_code is not None or input_scale is not None) and (
+            K <= 512 or (input_code is None and (weight_code is None or input.numel() > 512 * K))) and (
+                -(-(input.numel() // K) // 128) * -(-weight.shape[0] // 128) <= 256)
     if K > 0 and K % 64 == 0 and not (few_rows or transposed or one_launch) and _coded(
             input_code, input_scale, weight_code, weight_scale):
         # [M, K] rows against the weight decoded once
